@@ -8,7 +8,7 @@
 // both streams in one register tile under one running max and one running sum
 // is the online log-sum-exp merge of the two streams evaluated in place.
 //
-// Three kernels:
+// Four kernels:
 //  * attn_mfma_kernel<D>: bf16, head_dim 64/128/256, W <= 64, BS >= 64.
 //    Work unit = (batch, kv head, segment of 64-position chunks).  Keys of the
 //    current and previous 64-position page live in an LDS ring (K row-major,
@@ -16,6 +16,8 @@
 //    16 query positions and loops over the GQA group's query heads:
 //      S^T = K Q^T  and  O^T = V^T P^T  on v_mfma_f32_16x16x32_bf16,
 //    fp32 softmax with wavefront shuffles between the 4 lane groups.
+//  * page_attn_kernel<D> (page_attn.h): bf16, head_dim 64/128/256, the windows and block sizes that
+//    attn_mfma_kernel does not take; keys in LDS pages under a running softmax.
 //  * attn_f32_tile_kernel<D>: fp32, head_dim 64/128, W <= 64, GQA groups of at
 //    most 4, BS a multiple of 16; one workgroup per (batch, kv head, 16-query
 //    tile), keys staged in LDS, both products on v_mfma_f32_16x16x4_f32.
@@ -27,6 +29,7 @@
 
 #include "bfly_topology.h"
 #include "cache_update.h"
+#include "page_attn.h"
 
 namespace bfly {
 
@@ -1386,8 +1389,11 @@ attn_mfma_kernel(AttnArgs a_in, MfmaArgs m_in, int seg_chunks, int c_first_in, i
   }
 }
 
-// One attention launch: the MFMA kernel where its conditions hold, else the fp32 tile kernel
-// or the generic one.
+// Query blocks that 64 positions starting at a multiple of 64 can touch.
+static int chunk_blocks_max(int bs) { return bs % kPageRows == 0 ? 1 : kPageRows % bs == 0 ? kPageRows / bs : 62 / bs + 2; }
+
+// One attention launch: the MFMA kernel where its conditions hold, else the paged MFMA kernel
+// (bf16), the fp32 tile kernel or the generic one.
 static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, const char* what) {
   BFLY_CHECK_ARG(aligned16(a.q) && aligned16(a.out) && aligned16(a.k) && aligned16(a.v) && aligned16(a.ks) &&
                      aligned16(a.vs),
@@ -1450,6 +1456,26 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
       case 128: hipLaunchKernelGGL(attn_mfma_kernel<128>, grid, dim3(256), 0, stream, a, m, seg, (int)c_first, (int)nchunks, hper, NoBatch{}); break;
       default: hipLaunchKernelGGL(attn_mfma_kernel<256>, grid, dim3(MfmaCfg<256>::NTHR), 0, stream, a, m, seg, (int)c_first, (int)nchunks, hper, NoBatch{}); break;
     }
+  } else if (
+      // The paged kernel: its summary page holds 64 slots (the routed rows of every block that a
+      // 64-position chunk touches), a ring page may wrap once, positions are 32-bit.  It replaces the
+      // generic kernel wherever it can run: the whole one-shot call over 2 x 10007 tokens, 16 query
+      // heads over 4 of d 128, W 128 took 1711 us there and takes 119 us here, one decode row over a
+      // 128-token window 81 us (host work included) and 21 us.
+      dtype == BFLY_DTYPE_BF16 && contiguous && (a.d == 64 || a.d == 128 || a.d == 256) &&
+             a.W + a.kcap <= kGenericMaxKeys && chunk_blocks_max(a.bs) * (int64_t)a.kcap <= kPageRows &&
+             (a.ring == 0 || a.ring >= kPageRows) && a.q_pos0 >= 0 && a.q_pos0 + a.tq < (1 << 30) &&
+             a.kv_len < (1 << 30) && a.ring < (1 << 30) && a.nblocks >= 1 && a.nblocks * (int64_t)a.bs < (1 << 30) &&
+             a.batch * a.hkv <= 65535 && page_grid_fits(a.tq, a.batch, a.hq)) {
+    PageArgs g{};
+    g.q = a.q; g.k = a.k; g.v = a.v; g.ks = a.ks; g.vs = a.vs; g.out = a.out; g.nbr = a.nbr;
+    g.kv_rows = a.kv_rows; g.pool_rows = a.pool_rows;
+    g.batch = (int)a.batch; g.hq = a.hq; g.hkv = a.hkv; g.tq = (int)a.tq;
+    g.qlo = (int)a.q_pos0; g.qhi = (int)(a.q_pos0 + a.tq);
+    g.key_lo = (int)a.key_lo; g.kv_len = (int)a.kv_len; g.ring = (int)a.ring;
+    g.nblocks = (int)a.nblocks; g.nsum = (int)(a.nsum < a.nblocks ? a.nsum : a.nblocks);
+    g.kcap = a.kcap; g.bs = a.bs; g.W = a.W; g.token_cutoff = a.token_cutoff; g.scale = a.scale;
+    launch_page_attn<kPageFused>(g, a.d, stream);
   } else if (dtype == BFLY_DTYPE_F32 && contiguous && a.nbr != nullptr && a.W <= 64 && a.bs % 16 == 0 &&
              a.hq / a.hkv <= 4 &&
              (a.d == 64 || a.d == 128) && a.kcap >= 1 && a.kcap <= kF32MaxKcap &&

@@ -92,6 +92,8 @@ SIGNATURES = {
     "bfly_argmax_rows": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
     "bfly_argmax_rows_noalloc": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _vp]),
     "bfly_q4_gemv": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _vp, _vp]),
+    "bfly_q4_rows": (_int, [_vp, _i64, _vp, _vp, _i64, _i64, _int, _vp, _vp]),
+    "bfly_q4_rows_silu": (_int, [_vp, _i64, _vp, _vp, _i64, _i64, _int, _i64, _vp, _vp]),
     "bfly_q4_gemv_silu": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _i64, _vp, _vp]),
     "bfly_add_rms_norm_q4_gemv": (_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _i64, _i64, _int, _vp, _vp]),
     "bfly_add_rms_norm_q4_gemv_silu": (_int, [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _i64, _i64, _int, _i64, _vp,

@@ -107,6 +107,25 @@ int bfly_q4_gemv_silu(const void* x, const void* packed, const void* scale_bias,
                       int64_t in_features, int group, int64_t up_row_offset, void* out, hipStream_t stream);
 
 /*
+ * Device: the product of 1..32 rows x [rows, in_features] (bf16) with a quantized
+ * linear layer, out [rows, out_features] (bf16), from the 4-bit codes on the
+ * matrix cores: what bfly_q4_gemv computes for one row, fp32 sums in another
+ * order.  group 64, in_features a multiple of 256; x, packed and scale_bias
+ * 16-byte aligned.  Replaces the 4-bit affine quantized matmul of the reference's
+ * quantized projections (mlx.nn.QuantizedLinear as used at
+ * bna/integrations/qwen_mlx.py:1115-1157) for batched decode steps.
+ */
+int bfly_q4_rows(const void* x, int64_t rows, const void* packed, const void* scale_bias, int64_t out_features,
+                 int64_t in_features, int group, void* out, hipStream_t stream);
+
+/*
+ * Device: bfly_q4_gemv_silu for 1..32 rows (limits as bfly_q4_rows).  No
+ * counterpart in the reference's own code.
+ */
+int bfly_q4_rows_silu(const void* x, int64_t rows, const void* packed, const void* scale_bias, int64_t out_features,
+                      int64_t in_features, int group, int64_t up_row_offset, void* out, hipStream_t stream);
+
+/*
  * Device: bfly_add_rms_norm of one row followed by bfly_q4_gemv of the normed row, in
  * one launch: h_out = x + residual (bf16; skipped when residual and h_out are NULL),
  * out = W RMSNorm(h) * norm_weight, with the rounding points and summation order of

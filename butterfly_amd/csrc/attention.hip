@@ -615,18 +615,7 @@ struct MfmaArgs {
   int64_t upd_wgs;
 };
 
-// A batched streaming launch: the attention of up to kMaxUpdateParts consecutive chunks whose
-// cache updates are all done, one grid row band per chunk.  Each chunk keeps the arguments of
-// its own cache state (the counters right after its update), so its results are those of a
-// launch of its own.
-struct ChunkArgs {
-  const void* q;
-  void* out;
-  const void* k;          // the chunk's own keys and values, [batch x kv heads, tq, d]
-  const void* v;
-  int tq, qlo, qhi, key_lo, kv_len, nsum, nblocks, c_first, nchunks;
-  bfly_topology_t topo;
-};
+// A batched streaming launch (ChunkArgs, page_attn.h): one grid row band per chunk.
 struct ChunkBatch {
   int rows_per_chunk;     // grid rows of one chunk (batch x kv heads x head parts)
   int nch;                // chunks in the batch
@@ -1392,6 +1381,30 @@ attn_mfma_kernel(AttnArgs a_in, MfmaArgs m_in, int seg_chunks, int c_first_in, i
 // Query blocks that 64 positions starting at a multiple of 64 can touch.
 static int chunk_blocks_max(int bs) { return bs % kPageRows == 0 ? 1 : kPageRows % bs == 0 ? kPageRows / bs : 62 / bs + 2; }
 
+// Whether the paged kernel takes a bf16 launch over contiguous positions: its summary page holds 64
+// slots (the routed rows of every block that 64 positions touch), a ring page may wrap once,
+// positions are 32-bit.  It replaces the generic kernel wherever it can run: the one-shot call over
+// 2 x 10007 tokens, 16 query heads over 4 of d 128, W 128 took 1711 us there and takes 109 us here,
+// one decode row over a 128-token window 81 us (host work included) and 21 us.
+static bool page_path(const AttnArgs& a, int blocks) {
+  return (a.d == 64 || a.d == 128 || a.d == 256) && a.W + (int64_t)a.kcap <= kGenericMaxKeys &&
+         blocks * (int64_t)a.kcap <= kPageRows && (a.ring == 0 || a.ring >= kPageRows) && a.q_pos0 >= 0 &&
+         a.q_pos0 + a.tq < (1 << 30) && a.kv_len < (1 << 30) && a.ring < (1 << 30) && a.nblocks >= 1 &&
+         a.nblocks * (int64_t)a.bs < (1 << 30) && a.batch * a.hkv <= 65535 && page_grid_fits(a.tq, a.batch, a.hq);
+}
+
+static PageArgs page_args(const AttnArgs& a) {
+  PageArgs g{};
+  g.q = a.q; g.k = a.k; g.v = a.v; g.ks = a.ks; g.vs = a.vs; g.out = a.out; g.nbr = a.nbr;
+  g.kv_rows = a.kv_rows; g.pool_rows = a.pool_rows;
+  g.batch = (int)a.batch; g.hq = a.hq; g.hkv = a.hkv; g.tq = (int)a.tq;
+  g.qlo = (int)a.q_pos0; g.qhi = (int)(a.q_pos0 + a.tq);
+  g.key_lo = (int)a.key_lo; g.kv_len = (int)a.kv_len; g.ring = (int)a.ring;
+  g.nblocks = (int)a.nblocks; g.nsum = (int)(a.nsum < a.nblocks ? a.nsum : a.nblocks);
+  g.kcap = a.kcap; g.bs = a.bs; g.W = a.W; g.token_cutoff = a.token_cutoff; g.scale = a.scale;
+  return g;
+}
+
 // One attention launch: the MFMA kernel where its conditions hold, else the paged MFMA kernel
 // (bf16), the fp32 tile kernel or the generic one.
 static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, const char* what) {
@@ -1456,26 +1469,8 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
       case 128: hipLaunchKernelGGL(attn_mfma_kernel<128>, grid, dim3(256), 0, stream, a, m, seg, (int)c_first, (int)nchunks, hper, NoBatch{}); break;
       default: hipLaunchKernelGGL(attn_mfma_kernel<256>, grid, dim3(MfmaCfg<256>::NTHR), 0, stream, a, m, seg, (int)c_first, (int)nchunks, hper, NoBatch{}); break;
     }
-  } else if (
-      // The paged kernel: its summary page holds 64 slots (the routed rows of every block that a
-      // 64-position chunk touches), a ring page may wrap once, positions are 32-bit.  It replaces the
-      // generic kernel wherever it can run: the whole one-shot call over 2 x 10007 tokens, 16 query
-      // heads over 4 of d 128, W 128 took 1711 us there and takes 119 us here, one decode row over a
-      // 128-token window 81 us (host work included) and 21 us.
-      dtype == BFLY_DTYPE_BF16 && contiguous && (a.d == 64 || a.d == 128 || a.d == 256) &&
-             a.W + a.kcap <= kGenericMaxKeys && chunk_blocks_max(a.bs) * (int64_t)a.kcap <= kPageRows &&
-             (a.ring == 0 || a.ring >= kPageRows) && a.q_pos0 >= 0 && a.q_pos0 + a.tq < (1 << 30) &&
-             a.kv_len < (1 << 30) && a.ring < (1 << 30) && a.nblocks >= 1 && a.nblocks * (int64_t)a.bs < (1 << 30) &&
-             a.batch * a.hkv <= 65535 && page_grid_fits(a.tq, a.batch, a.hq)) {
-    PageArgs g{};
-    g.q = a.q; g.k = a.k; g.v = a.v; g.ks = a.ks; g.vs = a.vs; g.out = a.out; g.nbr = a.nbr;
-    g.kv_rows = a.kv_rows; g.pool_rows = a.pool_rows;
-    g.batch = (int)a.batch; g.hq = a.hq; g.hkv = a.hkv; g.tq = (int)a.tq;
-    g.qlo = (int)a.q_pos0; g.qhi = (int)(a.q_pos0 + a.tq);
-    g.key_lo = (int)a.key_lo; g.kv_len = (int)a.kv_len; g.ring = (int)a.ring;
-    g.nblocks = (int)a.nblocks; g.nsum = (int)(a.nsum < a.nblocks ? a.nsum : a.nblocks);
-    g.kcap = a.kcap; g.bs = a.bs; g.W = a.W; g.token_cutoff = a.token_cutoff; g.scale = a.scale;
-    launch_page_attn<kPageFused>(g, a.d, stream);
+  } else if (dtype == BFLY_DTYPE_BF16 && contiguous && page_path(a, chunk_blocks_max(a.bs))) {
+    launch_page_attn<kPageFused>(page_args(a), a.d, stream);
   } else if (dtype == BFLY_DTYPE_F32 && contiguous && a.nbr != nullptr && a.W <= 64 && a.bs % 16 == 0 &&
              a.hq / a.hkv <= 4 &&
              (a.d == 64 || a.d == 128) && a.kcap >= 1 && a.kcap <= kF32MaxKcap &&
@@ -1508,13 +1503,14 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
   return BFLY_OK;
 }
 
-// The attention of n (<= kMaxUpdateParts) consecutive streaming chunks in one launch (MFMA
-// path, neighbour rows from each chunk's topology): ch[j] holds chunk j's arguments as
+// The attention of n (<= kMaxUpdateParts) consecutive streaming chunks in one launch (neighbour
+// rows from each chunk's topology; `paged`: the paged kernel, for what the W <= 64 one does not
+// take): ch[j] holds chunk j's arguments as
 // bfly_stream_chunks builds them for a launch of its own; they differ only in the query range,
 // q / out and the cache state.  Optionally with a cache update on extra grid rows.  The grid
 // shape follows launch_attention's rules for the whole batch.
 static int launch_attention_batch(const AttnArgs* ch, const void* const* kin, const void* const* vin, int n,
-                                  bool from_inputs, hipStream_t stream, const char* what,
+                                  bool from_inputs, bool paged, hipStream_t stream, const char* what,
                                   const UpdateJob* upd = nullptr, int64_t upd_rows = 0) {
   BFLY_CHECK_ARG(n >= 1 && n <= kMaxUpdateParts, "%s: batch of %d chunks", what, n);
   const AttnArgs& a = ch[0];
@@ -1550,6 +1546,24 @@ static int launch_attention_batch(const AttnArgs* ch, const void* const* kin, co
     k.topo = c.topo;
   }
   const int64_t groups = a.batch * a.hkv;
+  if (paged) {
+    PageBatch pb{};
+    pb.nch = n;
+    pb.from_inputs = cb.from_inputs;
+    for (int j = 0; j < n; ++j) pb.c[j] = cb.c[j];
+    if (upd != nullptr) {
+      const int64_t ux = update_x(upd->n_blocks, upd->step - upd->append_from, upd->d, 8);
+      BFLY_CHECK_ARG(ux <= INT32_MAX && upd_rows <= 65535, "%s: grid too large", what);
+      pb.upd = *upd;
+      pb.upd_x = (int)ux;
+      pb.upd_rows = (int)upd_rows;
+      pb.upd_wgs = ux * upd_rows * 2;
+    }
+    BFLY_CHECK_ARG(nch_max * n * groups * (a.hq / a.hkv) + pb.upd_wgs < (1 << 30), "%s: grid too large", what);
+    launch_page_batch(page_args(a), pb, a.d, (int)nch_max, stream);
+    BFLY_CHECK_LAUNCH(what);
+    return BFLY_OK;
+  }
   int seg = 1;
   while (seg < kMaxSegChunks && (nch_max + 2 * seg - 1) / (2 * seg) * groups * n >= 512) seg *= 2;
   const int64_t nseg = (nch_max + seg - 1) / seg;
@@ -1683,8 +1697,9 @@ extern "C" int bfly_attend_cache(const void* q, int dtype, int64_t batch, int hq
 // per-chunk path.  Chunk c's attention and chunk c+1's update share one launch
 // when they touch disjoint ring slots and pool rows: the update writes positions
 // [P, P + len_{c+1}) (P = end of chunk c) and pool rows >= the summaries chunk c
-// reads, while chunk c's attention reads pages no lower than P - len_c - 2*64,
-// so len_c + len_{c+1} + 2*64 <= ring capacity keeps them apart.
+// reads, while chunk c's attention reads pages no lower than P - len_c - halo
+// (halo = the window's whole pages and one more), so len_c + len_{c+1} + halo <= ring
+// capacity keeps them apart.
 namespace {
 
 struct StreamCounters {
@@ -1774,13 +1789,20 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
     total += chunk_len[c];
   }
   const int kcap = 1 + local_window_blocks + partner_count + sink_count;
-  // the MFMA attention kernel is the one that builds neighbour rows from the topology
+  // the MFMA attention kernels are the ones that build neighbour rows from the topology
   const bool mfma_ok = dtype == BFLY_DTYPE_BF16 && window <= kPage && block_size >= kPage && 2 * kcap <= kSumSlots &&
                        (head_dim == 64 || head_dim == 128 || head_dim == 256) && scale > 0.f &&
                        ring_capacity >= kPage && ring_capacity >= block_size && total + 2 * kPage < INT32_MAX &&
                        ring_capacity < INT32_MAX && pool_capacity < INT32_MAX;
-  if (!mfma_ok) {
-    set_error("bfly_stream_chunks: configuration outside the MFMA attention path");
+  bool paged = false;
+  if (!mfma_ok && dtype == BFLY_DTYPE_BF16 && ring_capacity >= block_size && ring_capacity > 0) {
+    AttnArgs p{};      // every chunk's launch at once, for its limits
+    p.batch = batch; p.hq = hq; p.hkv = hkv; p.d = head_dim; p.tq = total; p.kv_len = total; p.ring = ring_capacity;
+    p.nblocks = (total + block_size - 1) / block_size; p.kcap = kcap; p.bs = block_size; p.W = window;
+    paged = page_path(p, chunk_blocks_max(block_size)) && pool_capacity < INT32_MAX;
+  }
+  if (!mfma_ok && !paged) {
+    set_error("bfly_stream_chunks: configuration outside the MFMA attention paths");
     return BFLY_ERR_UNSUPPORTED;
   }
   const int64_t rows = batch * hkv;
@@ -1795,27 +1817,50 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // batch that appends all its chunks and pools every block that becomes due over them (the
   // per-chunk counter steps run on the host; the pooled blocks are consecutive).  A batch's
   // update rides with the previous batch's attention when the two touch disjoint ring slots.
-  // Batch tokens are capped at (ring - 2*64) / 2 so that consecutive batches can share a
-  // launch; with a ring of a few chunks that is one chunk per batch, the per-chunk schedule.
+  // Batch tokens are capped at (ring - halo) / 2 so that consecutive batches can share a
+  // launch -- unless every chunk starts on a page boundary: the attention then reads the batch's own
+  // tokens from the inputs and the update copies only the tail it leaves, so a batch may hold more
+  // tokens than the ring, as long as no slot that is written is one that the update pools from or
+  // the attention's halo lies in (ring_disjoint).  With the default ring (1408 rows for 512-token chunks
+  // and 128-token windows) that is ten chunks a launch instead of one: 20011 tokens of d 256, 16
+  // query heads over 4, 1812 us a stream with a launch per chunk, 407 so.
   struct Batch {
     int64_t first = 0, count = 0, total = 0;
     AttnArgs args[kMaxUpdateParts];
     UpdateJob job{};
     StreamCounters end{};
     bool overflow = false;   // the last chunk exhausted the pool: its update runs, its attention not
+    int64_t ring_lo = 0;     // lowest position that the attention reads from the ring
     bool from_inputs = false;   // the attention reads the batch's own tokens from the chunk inputs
     int stop_rc = BFLY_OK;   // the chunk after the batch does not fit (its error)
   };
-  const int64_t budget = (ring_capacity - 2 * kPage) / 2;
+  const int64_t halo = (window - 1 + kPage - 1) / kPage * kPage + kPage;
+  const int64_t budget = (ring_capacity - halo) / 2;
+  // Wide batches leave the tokens below their tail out of the ring; the call's last launch copies
+  // those that its last ring_capacity positions hold (copy_rest), so that the whole ring is what one
+  // chunk per batch leaves.  A W <= 64 call whose chunks share batches under the length rule keeps
+  // that rule alone (its batches copy only their tails).
+  bool wide = true;
+  for (int64_t c = 0; !paged && c + 1 < n_chunks; ++c)
+    if (chunk_len[c] + chunk_len[c + 1] <= budget) wide = false;
+  const int64_t call_offset = s.offset;
   auto plan_batch = [&](const StreamCounters& s0, int64_t from, Batch& bt) -> int {
     bt = Batch{};
     bt.first = from;
     bt.end = s0;
+    // the chunks one by one, up to the cap; `take` is the longest prefix that one launch can hold
+    struct After {
+      StreamCounters st;
+      int64_t total, blocks;
+    } after[kMaxUpdateParts];
     StreamCounters st = s0;
-    int64_t blocks = 0;
-    for (int64_t c = from; c < n_chunks && bt.count < kMaxUpdateParts; ++c) {
+    int64_t blocks = 0, total_len = 0, count = 0, take = 0;
+    bool from_inputs = true;
+    // (the W <= 64 kernel stages the whole page before the queries' own)
+    const int64_t reach = window - 1 > kPage ? window - 1 : kPage;
+    const int64_t ring_lo = s0.offset > reach ? (s0.offset - reach) / kPage * kPage : 0;
+    for (int64_t c = from; c < n_chunks && count < kMaxUpdateParts; ++c) {
       const int64_t len = chunk_len[c];
-      if (bt.count > 0 && (bt.total + len > budget || s0.tail + bt.total + len > ring_capacity)) break;
       StreamCounters nx = st;
       PlannedUpdate pu{};
       const int prc = plan_update(nx, len, k[c], v[c], ring_k, ring_v, ring_capacity, pool_k, pool_v, pool_capacity,
@@ -1824,16 +1869,16 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
         bt.stop_rc = prc;
         break;
       }
-      if (pu.overflow && bt.count > 0) break;   // it starts the next batch, alone
+      if (pu.overflow && count > 0) break;   // it starts the next batch, alone
       const int frc = finish_update(nx, pu, len, pool_capacity, block_size, cache_window);
-      if (bt.count == 0) bt.job = pu.job;      // offset, first pooled block and slot of the batch
-      bt.job.k_part[bt.count] = k[c];
-      bt.job.v_part[bt.count] = v[c];
-      bt.job.part_end[bt.count] = bt.total + len;
+      if (count == 0) bt.job = pu.job;      // offset, first pooled block and slot of the batch
+      bt.job.k_part[count] = k[c];
+      bt.job.v_part[count] = v[c];
+      bt.job.part_end[count] = total_len + len;
       blocks += pu.n_new;
-      bt.total += len;
+      total_len += len;
       const int64_t nblocks = (nx.offset + block_size - 1) / block_size;
-      AttnArgs& a = bt.args[bt.count];
+      AttnArgs& a = bt.args[count];
       a = AttnArgs{};
       const int trc = bfly_topology_init(nblocks, layer_idx, partner_rule, local_window_blocks, sink_count,
                                          partner_count, &a.topo);
@@ -1845,29 +1890,80 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
       a.key_lo = nx.offset - nx.tail; a.kv_len = nx.offset;
       a.pool_rows = pool_capacity; a.nsum = nx.count; a.nblocks = nblocks;
       a.kcap = kcap; a.bs = block_size; a.W = window; a.scale = scale; a.token_cutoff = 1;
-      ++bt.count;
+      from_inputs = from_inputs && a.q_pos0 % kPage == 0;
+      after[count] = After{nx, total_len, blocks};
+      ++count;
       st = nx;
+      const int64_t tail_lo = nx.offset - nx.tail, w_lo = tail_lo > s0.offset ? tail_lo : s0.offset;
+      if (count == 1 || (total_len <= budget && s0.tail + total_len <= ring_capacity) ||
+          (wide && from_inputs &&
+           ring_disjoint(w_lo, nx.offset, ring_lo < s0.sum_off ? ring_lo : s0.sum_off, s0.offset, ring_capacity)))
+        take = count;
       if (pu.overflow) {              // finish_update reported it
         bt.overflow = true;
         (void)frc;
         break;
       }
+      if (!from_inputs && total_len > budget) break;   // no longer prefix can fit
     }
-    bt.end = st;
+    if (take < count) bt.stop_rc = BFLY_OK;            // the batch ends before the chunk that did not fit
+    bt.count = take;
+    bt.ring_lo = ring_lo;
+    if (take == 0) return BFLY_OK;
+    bt.end = after[take - 1].st;
+    bt.total = after[take - 1].total;
     bt.job.step = bt.total;
-    bt.job.n_blocks = (int)blocks;
-    bt.job.nparts = (int)bt.count;
+    bt.job.n_blocks = (int)after[take - 1].blocks;
+    bt.job.nparts = (int)take;
     // When every chunk of the batch starts on a page boundary, its attention reads the batch's
     // own tokens from the chunk inputs and only the tokens in the tail the batch leaves are
     // copied to the ring: every later read of the ring (pooling, attention windows, the cache's
     // views) lies in a later tail, which starts no earlier.
     bt.from_inputs = true;
-    for (int64_t j = 0; j < bt.count; ++j) bt.from_inputs = bt.from_inputs && bt.args[j].q_pos0 % kPage == 0;
-    const int64_t keep_from = st.offset - st.tail - bt.job.offset;
+    for (int64_t j = 0; j < take; ++j) bt.from_inputs = bt.from_inputs && bt.args[j].q_pos0 % kPage == 0;
+    const int64_t keep_from = bt.end.offset - bt.end.tail - bt.job.offset;
     bt.job.append_from = !bt.from_inputs || keep_from < 0 ? 0 : (keep_from > bt.total ? bt.total : keep_from);
     return BFLY_OK;
   };
+  // Whether `nx`'s update may run beside `cur`'s attention: by length, or because the attention reads
+  // only its halo from the ring and the update's appended tokens take other slots.
+  auto fuses = [&](const Batch& cur, const Batch& nx) {
+    return cur.total + nx.total + halo <= ring_capacity ||
+           (wide && cur.from_inputs && ring_disjoint(nx.job.offset + nx.job.append_from, nx.job.offset + nx.total, cur.ring_lo,
+                                             cur.job.offset, ring_capacity));
+  };
   auto launch_update = [&](const UpdateJob& j) -> int { return launch_update_job(j, rows, stream); };
+  // the tokens of chunks [0, done) below the tail that st leaves, of the last ring_capacity positions
+  auto copy_rest = [&](const StreamCounters& st, int64_t done) -> int {
+    const int64_t hi = st.offset - st.tail;
+    int64_t lo = st.offset - ring_capacity, pos = call_offset, c = 0;
+    if (!wide || lo >= hi) return BFLY_OK;
+    while (c < done && pos < hi) {
+      UpdateJob j{};
+      j.ring_k = ring_k; j.ring_v = ring_v; j.pool_k = pool_k; j.pool_v = pool_v;
+      j.ring = ring_capacity; j.pool_rows = pool_capacity; j.bs = block_size; j.d = head_dim;
+      j.offset = pos;
+      int64_t at = 0;
+      for (; c < done && j.nparts < kMaxUpdateParts && pos < hi; ++c) {
+        at += chunk_len[c];
+        pos += chunk_len[c];
+        if (pos <= lo && j.nparts == 0) {      // wholly below the range
+          j.offset = pos;
+          at = 0;
+          continue;
+        }
+        j.k_part[j.nparts] = k[c];
+        j.v_part[j.nparts] = v[c];
+        j.part_end[j.nparts++] = at;
+      }
+      if (j.nparts == 0) break;
+      j.step = (pos < hi ? pos : hi) - j.offset;
+      j.append_from = lo > j.offset ? lo - j.offset : 0;
+      const int rc = launch_update(j);
+      if (rc) return rc;
+    }
+    return BFLY_OK;
+  };
   if (n_chunks == 0) return BFLY_OK;
   // the first batch's update runs alone; every later one rides with the previous attention
   // when their ring slots are disjoint
@@ -1889,12 +1985,12 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
       nxt = Batch{};
       nxt.stop_rc = cur.stop_rc;
     }
-    if (nxt.count > 0 && cur.total + nxt.total + 2 * kPage <= ring_capacity) {
-      rc = launch_attention_batch(cur.args, cur.job.k_part, cur.job.v_part, (int)cur.count, cur.from_inputs,
+    if (nxt.count > 0 && fuses(cur, nxt)) {
+      rc = launch_attention_batch(cur.args, cur.job.k_part, cur.job.v_part, (int)cur.count, cur.from_inputs, paged,
                                   stream, "bfly_stream_chunks", &nxt.job, rows);
       if (rc) return rc;
     } else {
-      rc = launch_attention_batch(cur.args, cur.job.k_part, cur.job.v_part, (int)cur.count, cur.from_inputs,
+      rc = launch_attention_batch(cur.args, cur.job.k_part, cur.job.v_part, (int)cur.count, cur.from_inputs, paged,
                                   stream, "bfly_stream_chunks");
       if (rc) return rc;
       if (nxt.count > 0) {
@@ -1903,10 +1999,16 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
       }
     }
     *chunks_done = next_from;
-    if (nxt.count == 0) return nxt.stop_rc;
+    if (nxt.count == 0) {
+      rc = copy_rest(s, next_from);
+      return rc ? rc : nxt.stop_rc;
+    }
     s = nxt.end;
     publish(s);
-    if (nxt.overflow) return BFLY_ERR_CAPACITY;
+    if (nxt.overflow) {
+      rc = copy_rest(s, next_from + nxt.count);
+      return rc ? rc : BFLY_ERR_CAPACITY;
+    }
     cur = nxt;
   }
 }

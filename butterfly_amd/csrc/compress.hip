@@ -60,11 +60,16 @@ __global__ void __launch_bounds__(256) cache_update_kernel(UpdateJob u) {
 // loop's batches, whose new tokens may come from several chunk buffers.
 int launch_update_job(const UpdateJob& u, int64_t rows, hipStream_t stream) {
   BFLY_CHECK_ARG((u.d == 64 || u.d == 128 || u.d == 256) && rows > 0 && rows <= 65535, "update job shape");
-  // the due blocks lie inside the post-append tail: [offset + step - ring, offset + step)
-  BFLY_CHECK_ARG(u.n_blocks == 0 || (u.first_pos >= u.offset + u.step - u.ring &&
-                                     u.first_pos + (int64_t)u.n_blocks * u.bs <= u.offset + u.step),
-                 "update job: due blocks outside the tail after the append");
-  BFLY_CHECK_ARG(u.append_from >= 0 && u.append_from <= u.step, "update job: append_from outside the step");
+  BFLY_CHECK_ARG(u.append_from >= 0 && u.append_from <= u.step && u.step - u.append_from <= u.ring,
+                 "update job: append_from outside the step");
+  // the due blocks' old tokens are read from the ring beside the append: their slots are not the
+  // ones that the appended tokens take
+  const int64_t due_end = u.first_pos + (int64_t)u.n_blocks * u.bs;
+  BFLY_CHECK_ARG(u.n_blocks == 0 ||
+                     (due_end <= u.offset + u.step &&
+                      ring_disjoint(u.offset + u.append_from, u.offset + u.step, u.first_pos,
+                                    due_end < u.offset ? due_end : u.offset, u.ring)),
+                 "update job: due blocks on the appended tokens' slots");
   if (u.step == u.append_from && u.n_blocks == 0) return BFLY_OK;
   const int64_t ux = update_x(u.n_blocks, u.step - u.append_from, u.d, 8);
   BFLY_CHECK_ARG(ux <= INT32_MAX, "update job: grid too large");

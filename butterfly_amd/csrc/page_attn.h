@@ -30,7 +30,8 @@
 // head share their pages in an L2).
 #pragma once
 
-#include "bfly_common.h"
+#include "bfly_topology.h"
+#include "cache_update.h"
 
 namespace bfly {
 
@@ -60,6 +61,30 @@ struct PageArgs {
   // grid: items = chunks x (batch x hkv x head parts), item = (row, chunk), 8 contiguous runs
   int c_first, nchunks, nparts, per_xcd, items;
 };
+
+// A batched streaming launch: the attention of up to kMaxUpdateParts consecutive chunks whose
+// cache updates are all done, each with the arguments of its own cache state (the counters right
+// after its update), so its results are those of a launch of its own.
+struct ChunkArgs {
+  const void* q;
+  void* out;
+  const void* k;          // the chunk's own keys and values, [batch x kv heads, tq, d]
+  const void* v;
+  int tq, qlo, qhi, key_lo, kv_len, nsum, nblocks, c_first, nchunks;
+  bfly_topology_t topo;
+};
+// page_attn_kernel's batch.  Workgroups from attn_blocks on run a cache update instead
+// (cache_update_body over upd_x x upd_rows x K|V items, upd_wgs in all, one per 256 threads).
+struct PageBatch {
+  int nch;
+  int from_inputs;        // 1: every chunk starts on a page boundary; pages of the batch's own
+                          // tokens come from the chunk inputs (else every page from the ring)
+  int attn_blocks, upd_x, upd_rows;
+  int64_t upd_wgs;
+  UpdateJob upd;
+  ChunkArgs c[kMaxUpdateParts];
+};
+struct PageNoBatch {};
 
 template <int D, int NH>
 struct PageCfg {
@@ -93,8 +118,10 @@ __device__ __forceinline__ bool page_nonfinite(page_u32x4 x) {
   return t >= 0xff000000u;
 }
 
-template <int D, int HW, int NH, int MODE>
-__global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_attn_kernel(PageArgs a) {
+template <int D, int HW, int NH, int MODE, bool kBatch = false>
+__global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2)
+page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch> cb) {
+  PageArgs a = a_in;
   using C = PageCfg<D, NH>;
   constexpr int NTHR = C::NTHR, KP = C::KP, KSTEPS = C::KSTEPS, LD = C::LD, MT = D / 32;
   constexpr bool kWin = MODE == kPageFused || MODE == kPageSwa;
@@ -106,12 +133,45 @@ __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_
   __bf16* Ks = reinterpret_cast<__bf16*>(smem);
   __bf16* Vs = reinterpret_cast<__bf16*>(smem + C::K_BYTES);
 
+  static_assert(!kBatch || MODE == kPageFused, "batches are the streaming loop's");
+  if constexpr (kBatch) {
+    static_assert(C::LDS >= NH * 256 * 8 * 4, "pooling scratch aliases the staging tiles");
+    if ((int)blockIdx.x >= cb.attn_blocks) {
+      // a group of 256 threads whose item is past the end exits (it no longer counts at a barrier)
+      const int grp = (int)threadIdx.x >> 8;
+      const int64_t lin = (int64_t)((int)blockIdx.x - cb.attn_blocks) * NH + grp;
+      if (lin >= cb.upd_wgs) return;
+      const int64_t per_kv = (int64_t)cb.upd_x * cb.upd_rows;
+      const int kv = (int)(lin / per_kv);
+      const int64_t r = lin - kv * per_kv, urow = r / cb.upd_x;
+      cache_update_body<__bf16, 8>(cb.upd, r - urow * cb.upd_x, urow, kv, reinterpret_cast<float*>(smem) + grp * 256 * 8,
+                                   (int)threadIdx.x & 255);
+      return;
+    }
+  }
   // workgroups go round-robin over the 8 XCDs: XCD x takes items x per_xcd .. , whose consecutive
   // chunks share pages in its L2
   const int item = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
   if (item >= a.items) return;   // the whole workgroup
-  const int row = item / a.nchunks;
-  const int chunk = a.c_first + item - row * a.nchunks;
+  int row = item / a.nchunks;
+  int chunk = a.c_first + item - row * a.nchunks;
+  if constexpr (kBatch) {
+    // item = (row, chunk of the batch, 64 positions): a.nchunks is the longest chunk's
+    const int c64 = item - row * a.nchunks, zc = row % cb.nch;
+    row /= cb.nch;
+    const ChunkArgs& ck = cb.c[zc];
+    if (c64 >= ck.nchunks) return;
+    chunk = ck.c_first + c64;
+    a.q = ck.q;
+    a.out = ck.out;
+    a.tq = ck.tq;
+    a.qlo = ck.qlo;
+    a.qhi = ck.qhi;
+    a.key_lo = ck.key_lo;
+    a.kv_len = ck.kv_len;
+    a.nsum = ck.nsum;
+    a.nblocks = ck.nblocks;
+  }
   const int bh = row / a.nparts, hpart = row - bh * a.nparts;
   const int bi = bh / a.hkv, kvh = bh - bi * a.hkv;
   const int gsz = a.hq / a.hkv;
@@ -169,41 +229,53 @@ __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_
 
   page_u32x4 kst[LD], vst[LD];
   int cand[LD];      // kRouted: the staged rows' list entries
-  const page_u32x4 zero4 = {0u, 0u, 0u, 0u};
-  // Loads are unconditional (row 0 stands in for a row that does not exist) and the value is
-  // zeroed afterwards, so no branch splits the batch.
-  auto put = [&](int j, const __bf16* kr, const __bf16* vr, int64_t r, int pc, bool ok) {
-    const page_u32x4 x = *reinterpret_cast<const page_u32x4*>(kr + (ok ? r : 0) * D + pc * 8);
-    const page_u32x4 y = *reinterpret_cast<const page_u32x4*>(vr + (ok ? r : 0) * D + pc * 8);
-    kst[j] = ok ? x : zero4;
-    vst[j] = ok ? y : zero4;
-  };
+  // Loads are unconditional: row 0 stands in for a row that does not exist.  Such a row is masked
+  // in the scores, and no value of it is needed (its V takes weight 0; were it infinite, the page
+  // would be summed key by key), so nothing waits for the loads before the page is stored.
   auto fetch = [&](int it) {
+    int rr[LD];
+    const __bf16 *kr = ksb, *vr = vsb;
     if (kWin && it < nwin) {
       const int p0 = (chunk - it) * kPageRows;
-      int r0 = p0 - a.key_lo;
+      int r0 = p0 - a.key_lo, wrap = a.ring;
       if (a.ring) r0 = (int)((unsigned)p0 % (unsigned)a.ring);   // p0 >= 0
+      kr = kb;
+      vr = vb;
+      if constexpr (kBatch) {
+        if (cb.from_inputs && p0 >= cb.c[0].qlo) {
+          // the chunk that holds the page (it lies in one), by selects over the slots (uniform)
+          const void *kc = cb.c[0].k, *vc = cb.c[0].v;
+          int lo = cb.c[0].qlo, len = cb.c[0].tq;
+#pragma unroll
+          for (int j = 1; j < kMaxUpdateParts; ++j) {
+            const bool in = j < cb.nch && p0 >= cb.c[j].qlo;
+            kc = in ? cb.c[j].k : kc;
+            vc = in ? cb.c[j].v : vc;
+            lo = in ? cb.c[j].qlo : lo;
+            len = in ? cb.c[j].tq : len;
+          }
+          kr = reinterpret_cast<const __bf16*>(kc) + (int64_t)bh * len * D;
+          vr = reinterpret_cast<const __bf16*>(vc) + (int64_t)bh * len * D;
+          r0 = p0 - lo;      // rows past the chunk's end are past kv_len, the attended chunk's end
+          wrap = 0;
+        }
+      }
 #pragma unroll
       for (int j = 0; j < LD; ++j) {
-        const int i = tid + j * NTHR, r = i / C::PIECES, pc = i % C::PIECES;
+        const int r = (tid + j * NTHR) / C::PIECES;
         const bool ok = p0 + r >= a.key_lo && p0 + r < a.kv_len;
-        int rr = r0 + r;
-        if (a.ring && rr >= a.ring) rr -= a.ring;
-        put(j, kb, vb, rr, pc, ok);
+        int x = r0 + r;
+        if (wrap && x >= wrap) x -= wrap;
+        rr[j] = ok ? x : 0;
       }
     } else if constexpr (MODE == kPageFused) {
 #pragma unroll
-      for (int j = 0; j < LD; ++j) {
-        const int i = tid + j * NTHR, r = i / C::PIECES, pc = i % C::PIECES;
-        const int n = s_n[r];
-        put(j, ksb, vsb, n, pc, n >= 0);
-      }
+      for (int j = 0; j < LD; ++j) rr[j] = max(s_n[(tid + j * NTHR) / C::PIECES], 0);
     } else if constexpr (MODE == kPageDense) {
 #pragma unroll
       for (int j = 0; j < LD; ++j) {
-        const int i = tid + j * NTHR, r = i / C::PIECES, pc = i % C::PIECES;
-        const int n = it * kPageRows + r;
-        put(j, ksb, vsb, n, pc, n < nslots);
+        const int n = it * kPageRows + (tid + j * NTHR) / C::PIECES;
+        rr[j] = n < nslots ? n : 0;
       }
     } else if constexpr (MODE == kPageRouted) {
       const int li = it / per_list, bb = bA + li, s0 = (it - li * per_list) * kPageRows;
@@ -213,16 +285,35 @@ __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_
         const int s = s0 + (tid + j * NTHR) / C::PIECES;
         const int n = list[min(s, a.kcap - 1)];
         cand[j] = s < a.kcap && n >= 0 && n < bb && n < a.nsum ? n : -1;
+        rr[j] = max(cand[j], 0);
       }
-#pragma unroll
-      for (int j = 0; j < LD; ++j) put(j, ksb, vsb, cand[j], (tid + j * NTHR) % C::PIECES, cand[j] >= 0);
     }
+#pragma unroll
+    for (int j = 0; j < LD; ++j)
+      kst[j] = *reinterpret_cast<const page_u32x4*>(kr + (int64_t)rr[j] * D + (tid + j * NTHR) % C::PIECES * 8);
+#pragma unroll
+    for (int j = 0; j < LD; ++j)
+      vst[j] = *reinterpret_cast<const page_u32x4*>(vr + (int64_t)rr[j] * D + (tid + j * NTHR) % C::PIECES * 8);
   };
 
   if (npages > 0 && (MODE != kPageFused || nwin > 0)) fetch(0);
   if (tid < 2) s_bad[tid] = 0;
   if constexpr (MODE == kPageFused) {
-    if (tid < kPageRows) {
+    if constexpr (kBatch) {
+      // no table: thread t < blocks writes the row of block bA + t (neighbor_row, the table
+      // builder's), the first wave clears the slots past them
+      if (tid >= nslots && tid < kPageRows) s_n[tid] = -1;
+      const int bb = bA + tid;
+      if (bb <= bB) {
+        int32_t* list = s_n + tid * a.kcap;
+        const int len = neighbor_row(bb, a.nblocks, cb.c[(item / a.nchunks) % cb.nch].topo, list, a.kcap);
+        for (int j = 0; j < a.kcap; ++j) {
+          const int n = j < len ? list[j] : -1;
+          list[j] = n < bb && n < a.nsum ? n : -1;
+          s_b[tid * a.kcap + j] = bb;
+        }
+      }
+    } else if (tid < kPageRows) {
       const int bb = bA + tid / a.kcap;
       int n = -1;
       if (tid < nslots) {
@@ -308,30 +399,33 @@ __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_
             s[u][tt] = acc * sl2;
           }
         }
-        unsigned okm = 0xffu;            // bit 4 tt + i: key 16 tt + 4 lg + i of the group
-        if (!all) {
-          okm = 0u;
+        // is key `slot` of the page one that this lane's row attends to
+        auto win_ok = [&](int slot) { return p0 + slot >= wlo && p0 + slot <= qp; };
+        auto sum_ok = [&](int slot) {
+          if constexpr (MODE == kPageFused) {
+            const int n = s_n[slot];
+            return n >= 0 && s_b[slot] == qblk && (n + 1) * a.bs <= qcut;
+          } else if constexpr (MODE == kPageDense) {
+            const int n = it * kPageRows + slot;
+            return n < nslots && n < qblk;
+          } else {
+            return s_n[slot] >= 0 && bA + it / per_list == qblk;
+          }
+        };
+        auto mask = [&](auto ok_of) {
 #pragma unroll
           for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const int slot = 32 * pr + 16 * tt + 4 * lg + i;
-              bool ok;
-              if (win) {
-                ok = p0 + slot >= wlo && p0 + slot <= qp;
-              } else if constexpr (MODE == kPageFused) {
-                const int n = s_n[slot];
-                ok = n >= 0 && s_b[slot] == qblk && (n + 1) * a.bs <= qcut;
-              } else if constexpr (MODE == kPageDense) {
-                const int n = it * kPageRows + slot;
-                ok = n < nslots && n < qblk;
-              } else {
-                ok = s_n[slot] >= 0 && bA + it / per_list == qblk;
-              }
-              okm |= ok ? 1u << (4 * tt + i) : 0u;
+              const bool ok = ok_of(32 * pr + 16 * tt + 4 * lg + i);
 #pragma unroll
               for (int u = 0; u < HW; ++u) s[u][tt][i] = ok ? s[u][tt][i] : -INFINITY;
             }
+        };
+        if (win) {
+          if (!all) mask(win_ok);
+        } else {
+          mask(sum_ok);
         }
         bf16x8 hi[HW], lo[HW];
 #pragma unroll
@@ -379,7 +473,7 @@ __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_
               }
             }
         } else {
-          // key by key, only those the row attends to (a key's weight and mask from the lane group
+          // key by key, only those the row attends to (a key's weight from the lane group
           // that scored it): O[d] of tile (mt, half) in lane (lg, lq) is d = 32 mt + 8 lg + 4 half + i
 #pragma unroll
           for (int tt = 0; tt < 2; ++tt)
@@ -387,8 +481,8 @@ __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2) page_
             for (int i = 0; i < 4; ++i)
 #pragma unroll 1
               for (int src = 0; src < 4; ++src) {
-                const bool take = (__shfl((int)okm, lq + 16 * src) >> (4 * tt + i)) & 1;
                 const int key = 32 * pr + 16 * tt + 4 * src + i;
+                const bool take = win ? win_ok(key) : sum_ok(key);
 #pragma unroll
                 for (int u = 0; u < HW; ++u) {
                   const float p = __shfl(s[u][tt][i], lq + 16 * src);
@@ -470,7 +564,7 @@ static inline void launch_page_attn(PageArgs a, int d, hipStream_t stream) {
     a.nparts = (gsz + heads - 1) / heads;
     a.items = (int)(units * a.nparts);
     a.per_xcd = (a.items + 7) / 8;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * a.per_xcd)), dim3(threads), 0, stream, a);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * a.per_xcd)), dim3(threads), 0, stream, a, PageNoBatch{});
   };
   if constexpr (MODE == kPageRouted) {
     if (d == 64) go(page_attn_kernel<64, 1, 1, MODE>, 1, 256);
@@ -491,6 +585,27 @@ static inline void launch_page_attn(PageArgs a, int d, hipStream_t stream) {
       go(page_attn_kernel<256, 1, 2, MODE>, 2, 512);   // (with one head the other waves only stage)
     }
   }
+}
+
+// The attention of a batch of streaming chunks (cb.c[0 .. nch), cb.upd and its item counts filled) and,
+// with upd_wgs > 0, the next batch's cache update on workgroups behind them.
+static inline void launch_page_batch(PageArgs a, PageBatch cb, int d, int nchunks_max, hipStream_t stream) {
+  const int gsz = a.hq / a.hkv;
+  auto go = [&](auto kernel, int heads, int nh) {
+    a.c_first = 0;
+    a.nchunks = nchunks_max;
+    a.nparts = (gsz + heads - 1) / heads;
+    a.items = nchunks_max * cb.nch * a.batch * a.hkv * a.nparts;
+    a.per_xcd = (a.items + 7) / 8;
+    cb.attn_blocks = 8 * a.per_xcd;
+    const int64_t extra = (cb.upd_wgs + nh - 1) / nh;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(cb.attn_blocks + extra)), dim3(256 * nh), 0, stream, a, cb);
+  };
+  if (d == 256) go(page_attn_kernel<256, 1, 2, kPageFused, true>, 2, 2);
+  else if (d == 128 && gsz > 1) go(page_attn_kernel<128, 2, 1, kPageFused, true>, 2, 1);
+  else if (d == 128) go(page_attn_kernel<128, 1, 1, kPageFused, true>, 1, 1);
+  else if (gsz > 1) go(page_attn_kernel<64, 2, 1, kPageFused, true>, 2, 1);
+  else go(page_attn_kernel<64, 1, 1, kPageFused, true>, 1, 1);
 }
 
 // Items of the widest split (one head per workgroup) that the kernel's 32-bit grid arithmetic takes.

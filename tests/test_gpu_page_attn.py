@@ -204,3 +204,47 @@ def test_streams(b, hq, hkv, t, d, w, bs, factor):
     _stream_check(bf.compressed_stream_attention(qd, ks.cuda(), vs.cuda(), block_size=bs, scale=scale,
                                                  routed_indices=routed.cuda()),
                   oa.compressed_stream(qf, rep(ks), rep(vs), block_size=bs, scale=scale, routed_indices=routed))
+
+
+# chunk lengths, ring (max_chunk), windows and heads: the default ring with page-aligned chunks (batches
+# longer than the ring, some lengths cut where slots would collide), chunks off the page grid, an
+# attention window above the cache's, blocks below a page, the W <= 64 kernel with a small ring
+STREAMS = [
+    # d, hq, hkv, W, cache W, bs, max_chunk, chunk lengths
+    (256, 16, 4, 128, 128, 128, 512, [512] * 23 + [300]),
+    (128, 4, 4, 128, 128, 128, 512, [256] * 31),
+    (128, 8, 2, 128, 128, 128, 320, [320, 192, 64, 320, 320, 128] * 4 + [17]),
+    (64, 8, 1, 100, 64, 64, 200, [64] * 40),
+    (64, 2, 2, 128, 128, 128, 512, [100, 33, 512, 3, 200, 512, 511] * 2),
+    (128, 4, 2, 70, 96, 32, 256, [192] * 15),
+    (128, 8, 2, 64, 64, 128, 512, [512] * 14),
+    (256, 8, 2, 33, 64, 64, 256, [128] * 29 + [40]),
+    (64, 4, 1, 64, 64, 128, 448, [448, 64, 384] * 6),
+]
+
+
+@pytest.mark.parametrize("case", STREAMS, ids=lambda c: "-".join(str(x) for x in c[:7]))
+def test_stream_batches_match_single_chunks(case):
+    """chunked_prefill (batched launches, updates beside attention) against one core call per chunk:
+    outputs, tail, pools and counters bit for bit."""
+    d, hq, hkv, w, cw, bs, max_chunk, lens = case
+    cfg = bf.compressed_butterfly_config(block_size=bs, compressed_local_window_tokens=w, block_partner_rule="xor")
+    g = torch.Generator(device="cuda").manual_seed(5)
+    chunks = [tuple(torch.randn(2, h, n, d, generator=g, device="cuda").bfloat16() for h in (hq, hkv, hkv)) for n in lens]
+    caches = [bf.CompressedKVCache(block_size=bs, local_window_tokens=cw, max_kv_size=sum(lens), max_chunk_size=max_chunk)
+              for _ in range(2)]
+    core = bf.ButterflyAttentionCore(cfg, 5)
+    got = bf.chunked_prefill(core, chunks, caches[0])
+    assert core.last_profile.notes.get("native_chunk_loop")
+    want = [core(*c, caches[1]) for c in chunks]
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), i
+    x, y = caches
+    assert (x.offset, x.tail_size, x.summary_count, x.summary_offset) == \
+        (y.offset, y.tail_size, y.summary_count, y.summary_offset)
+    for a, b in zip(x.get_compressed_state()[:4], y.get_compressed_state()[:4]):
+        assert torch.equal(a, b)
+    # the whole ring, but where the W <= 64 batches of several short chunks copy only their tails
+    if w > 64 or min(a + b for a, b in zip(lens[1:], lens[2:])) > (x.tail_capacity - 128) // 2:
+        assert torch.equal(x.ring_state().ring_k, y.ring_state().ring_k)
+        assert torch.equal(x.ring_state().ring_v, y.ring_state().ring_v)

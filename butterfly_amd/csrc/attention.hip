@@ -29,7 +29,7 @@
 
 #include "bfly_topology.h"
 #include "cache_update.h"
-#include "page_attn.h"
+#include "win_attn.h"
 
 namespace bfly {
 
@@ -1470,7 +1470,11 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
       default: hipLaunchKernelGGL(attn_mfma_kernel<256>, grid, dim3(MfmaCfg<256>::NTHR), 0, stream, a, m, seg, (int)c_first, (int)nchunks, hper, NoBatch{}); break;
     }
   } else if (dtype == BFLY_DTYPE_BF16 && contiguous && page_path(a, chunk_blocks_max(a.bs))) {
-    launch_page_attn<kPageFused>(page_args(a), a.d, stream);
+    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, a.key_lo, a.kv_len, a.ring) &&
+        win_fills(a.q_pos0, a.tq, a.batch, a.hq, a.hkv))
+      launch_win_attn<kPageFused>(page_args(a), a.d, stream);
+    else
+      launch_page_attn<kPageFused>(page_args(a), a.d, stream);
   } else if (dtype == BFLY_DTYPE_F32 && contiguous && a.nbr != nullptr && a.W <= 64 && a.bs % 16 == 0 &&
              a.hq / a.hkv <= 4 &&
              (a.d == 64 || a.d == 128) && a.kcap >= 1 && a.kcap <= kF32MaxKcap &&
@@ -1560,7 +1564,10 @@ static int launch_attention_batch(const AttnArgs* ch, const void* const* kin, co
       pb.upd_wgs = ux * upd_rows * 2;
     }
     BFLY_CHECK_ARG(nch_max * n * groups * (a.hq / a.hkv) + pb.upd_wgs < (1 << 30), "%s: grid too large", what);
-    launch_page_batch(page_args(a), pb, a.d, (int)nch_max, stream);
+    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, 0, 1, a.ring))
+      launch_win_batch(page_args(a), pb, a.d, (int)nch_max, stream);
+    else
+      launch_page_batch(page_args(a), pb, a.d, (int)nch_max, stream);
     BFLY_CHECK_LAUNCH(what);
     return BFLY_OK;
   }

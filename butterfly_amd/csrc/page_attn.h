@@ -118,6 +118,102 @@ __device__ __forceinline__ bool page_nonfinite(page_u32x4 x) {
   return t >= 0xff000000u;
 }
 
+// This workgroup's (row, 64-position chunk) item, and in a batch its chunk's arguments put into `a` and its
+// index into zc; false for a workgroup past the items.  Workgroups go round-robin over the 8 XCDs: XCD x
+// takes items x per_xcd .. , whose consecutive chunks share pages in its L2.
+template <bool kBatch>
+__device__ __forceinline__ bool page_unit(PageArgs& a, const std::conditional_t<kBatch, PageBatch, PageNoBatch>& cb,
+                                          int& row, int& chunk, int& zc) {
+  const int item = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
+  if (item >= a.items) return false;   // the whole workgroup
+  row = item / a.nchunks;
+  chunk = a.c_first + item - row * a.nchunks;
+  zc = 0;
+  if constexpr (kBatch) {
+    // item = (row, chunk of the batch, 64 positions): a.nchunks is the longest chunk's
+    const int c64 = item - row * a.nchunks;
+    zc = row % cb.nch;
+    row /= cb.nch;
+    const ChunkArgs& ck = cb.c[zc];
+    if (c64 >= ck.nchunks) return false;
+    chunk = ck.c_first + c64;
+    a.q = ck.q;
+    a.out = ck.out;
+    a.tq = ck.tq;
+    a.qlo = ck.qlo;
+    a.qhi = ck.qhi;
+    a.key_lo = ck.key_lo;
+    a.kv_len = ck.kv_len;
+    a.nsum = ck.nsum;
+    a.nblocks = ck.nblocks;
+  }
+  return true;
+}
+
+// A batch's update work of this workgroup (blockIdx.x >= attn_blocks); `part`: 256 * 8 floats of LDS per
+// 256 threads.  A group of 256 threads whose item is past the end exits (it no longer counts at a barrier).
+template <int NH>
+__device__ __forceinline__ void page_update(const PageBatch& cb, float* part) {
+  const int grp = (int)threadIdx.x >> 8;
+  const int64_t lin = (int64_t)((int)blockIdx.x - cb.attn_blocks) * NH + grp;
+  if (lin >= cb.upd_wgs) return;
+  const int64_t per_kv = (int64_t)cb.upd_x * cb.upd_rows;
+  const int kv = (int)(lin / per_kv);
+  const int64_t r = lin - kv * per_kv, urow = r / cb.upd_x;
+  cache_update_body<__bf16, 8>(cb.upd, r - urow * cb.upd_x, urow, kv, part + grp * 256 * 8, (int)threadIdx.x & 255);
+}
+
+// The batch chunk that holds the page of positions p0 .. (it lies in one), by selects over the slots
+// (uniform): its keys and values [batch x kv heads, len, d], the first of them position lo.
+__device__ __forceinline__ void page_input(const PageBatch& cb, int p0, const void*& k, const void*& v, int& lo,
+                                           int& len) {
+  k = cb.c[0].k;
+  v = cb.c[0].v;
+  lo = cb.c[0].qlo;
+  len = cb.c[0].tq;
+#pragma unroll
+  for (int j = 1; j < kMaxUpdateParts; ++j) {
+    const bool in = j < cb.nch && p0 >= cb.c[j].qlo;
+    k = in ? cb.c[j].k : k;
+    v = in ? cb.c[j].v : v;
+    lo = in ? cb.c[j].qlo : lo;
+    len = in ? cb.c[j].tq : len;
+  }
+}
+
+// The routed summary slots of query blocks bA .. bB into LDS: slot s holds entry s % kcap of block
+// bA + s / kcap's row (s_n: the block, -1 where there is none before the row's or not yet summarised;
+// s_b: the row's block), `cap` slots in all.
+template <bool kBatch>
+__device__ __forceinline__ void page_slots(const PageArgs& a, const std::conditional_t<kBatch, PageBatch, PageNoBatch>& cb,
+                                           int zc, int bA, int bB, int cap, int* s_n, int* s_b) {
+  const int tid = threadIdx.x, nslots = (bB - bA + 1) * a.kcap;
+  if constexpr (kBatch) {
+    // no table: thread t < blocks writes the row of block bA + t (neighbor_row, the table
+    // builder's), the first wave clears the slots past them
+    if (tid >= nslots && tid < cap) s_n[tid] = -1;
+    const int bb = bA + tid;
+    if (bb <= bB) {
+      int32_t* list = s_n + tid * a.kcap;
+      const int len = neighbor_row(bb, a.nblocks, cb.c[zc].topo, list, a.kcap);
+      for (int j = 0; j < a.kcap; ++j) {
+        const int n = j < len ? list[j] : -1;
+        list[j] = n < bb && n < a.nsum ? n : -1;
+        s_b[tid * a.kcap + j] = bb;
+      }
+    }
+  } else if (tid < cap) {
+    const int bb = bA + tid / a.kcap;
+    int n = -1;
+    if (tid < nslots) {
+      n = a.nbr[(int64_t)bb * a.kcap + tid % a.kcap];
+      if (n >= bb || n >= a.nsum) n = -1;
+    }
+    s_n[tid] = n;
+    s_b[tid] = bb;
+  }
+}
+
 template <int D, int HW, int NH, int MODE, bool kBatch = false>
 __global__ void __launch_bounds__(256 * NH, (HW == 1 && D <= 128) ? 3 : 2)
 page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch> cb) {
@@ -137,41 +233,12 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
   if constexpr (kBatch) {
     static_assert(C::LDS >= NH * 256 * 8 * 4, "pooling scratch aliases the staging tiles");
     if ((int)blockIdx.x >= cb.attn_blocks) {
-      // a group of 256 threads whose item is past the end exits (it no longer counts at a barrier)
-      const int grp = (int)threadIdx.x >> 8;
-      const int64_t lin = (int64_t)((int)blockIdx.x - cb.attn_blocks) * NH + grp;
-      if (lin >= cb.upd_wgs) return;
-      const int64_t per_kv = (int64_t)cb.upd_x * cb.upd_rows;
-      const int kv = (int)(lin / per_kv);
-      const int64_t r = lin - kv * per_kv, urow = r / cb.upd_x;
-      cache_update_body<__bf16, 8>(cb.upd, r - urow * cb.upd_x, urow, kv, reinterpret_cast<float*>(smem) + grp * 256 * 8,
-                                   (int)threadIdx.x & 255);
+      page_update<NH>(cb, reinterpret_cast<float*>(smem));
       return;
     }
   }
-  // workgroups go round-robin over the 8 XCDs: XCD x takes items x per_xcd .. , whose consecutive
-  // chunks share pages in its L2
-  const int item = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
-  if (item >= a.items) return;   // the whole workgroup
-  int row = item / a.nchunks;
-  int chunk = a.c_first + item - row * a.nchunks;
-  if constexpr (kBatch) {
-    // item = (row, chunk of the batch, 64 positions): a.nchunks is the longest chunk's
-    const int c64 = item - row * a.nchunks, zc = row % cb.nch;
-    row /= cb.nch;
-    const ChunkArgs& ck = cb.c[zc];
-    if (c64 >= ck.nchunks) return;
-    chunk = ck.c_first + c64;
-    a.q = ck.q;
-    a.out = ck.out;
-    a.tq = ck.tq;
-    a.qlo = ck.qlo;
-    a.qhi = ck.qhi;
-    a.key_lo = ck.key_lo;
-    a.kv_len = ck.kv_len;
-    a.nsum = ck.nsum;
-    a.nblocks = ck.nblocks;
-  }
+  int row, chunk, zc;
+  if (!page_unit<kBatch>(a, cb, row, chunk, zc)) return;
   const int bh = row / a.nparts, hpart = row - bh * a.nparts;
   const int bi = bh / a.hkv, kvh = bh - bi * a.hkv;
   const int gsz = a.hq / a.hkv;
@@ -243,17 +310,9 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
       vr = vb;
       if constexpr (kBatch) {
         if (cb.from_inputs && p0 >= cb.c[0].qlo) {
-          // the chunk that holds the page (it lies in one), by selects over the slots (uniform)
-          const void *kc = cb.c[0].k, *vc = cb.c[0].v;
-          int lo = cb.c[0].qlo, len = cb.c[0].tq;
-#pragma unroll
-          for (int j = 1; j < kMaxUpdateParts; ++j) {
-            const bool in = j < cb.nch && p0 >= cb.c[j].qlo;
-            kc = in ? cb.c[j].k : kc;
-            vc = in ? cb.c[j].v : vc;
-            lo = in ? cb.c[j].qlo : lo;
-            len = in ? cb.c[j].tq : len;
-          }
+          const void *kc, *vc;
+          int lo, len;
+          page_input(cb, p0, kc, vc, lo, len);
           kr = reinterpret_cast<const __bf16*>(kc) + (int64_t)bh * len * D;
           vr = reinterpret_cast<const __bf16*>(vc) + (int64_t)bh * len * D;
           r0 = p0 - lo;      // rows past the chunk's end are past kv_len, the attended chunk's end
@@ -299,30 +358,7 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
   if (npages > 0 && (MODE != kPageFused || nwin > 0)) fetch(0);
   if (tid < 2) s_bad[tid] = 0;
   if constexpr (MODE == kPageFused) {
-    if constexpr (kBatch) {
-      // no table: thread t < blocks writes the row of block bA + t (neighbor_row, the table
-      // builder's), the first wave clears the slots past them
-      if (tid >= nslots && tid < kPageRows) s_n[tid] = -1;
-      const int bb = bA + tid;
-      if (bb <= bB) {
-        int32_t* list = s_n + tid * a.kcap;
-        const int len = neighbor_row(bb, a.nblocks, cb.c[(item / a.nchunks) % cb.nch].topo, list, a.kcap);
-        for (int j = 0; j < a.kcap; ++j) {
-          const int n = j < len ? list[j] : -1;
-          list[j] = n < bb && n < a.nsum ? n : -1;
-          s_b[tid * a.kcap + j] = bb;
-        }
-      }
-    } else if (tid < kPageRows) {
-      const int bb = bA + tid / a.kcap;
-      int n = -1;
-      if (tid < nslots) {
-        n = a.nbr[(int64_t)bb * a.kcap + tid % a.kcap];
-        if (n >= bb || n >= a.nsum) n = -1;
-      }
-      s_n[tid] = n;
-      s_b[tid] = bb;
-    }
+    page_slots<kBatch>(a, cb, zc, bA, bB, kPageRows, s_n, s_b);
   }
   __syncthreads();   // s_bad and the summary slots
   if (MODE == kPageFused && nwin == 0 && npages > 0) fetch(0);

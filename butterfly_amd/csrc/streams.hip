@@ -16,7 +16,7 @@
 // groups of 64 (one per lane) with a running max and rescaled accumulators, so
 // any window or summary count works in constant LDS; the result equals the
 // reference's single-pass softmax up to fp32 rounding.
-#include "page_attn.h"
+#include "win_attn.h"
 
 namespace bfly {
 
@@ -228,7 +228,9 @@ static int launch_stream(const StreamArgs& a, int dtype, hipStream_t stream, con
     g.qlo = 0; g.qhi = (int)a.tq; g.key_lo = 0; g.kv_len = (int)a.tq; g.ring = 0;
     g.nblocks = (int)((a.tq + a.bs - 1) / a.bs); g.nsum = (int)a.nsum; g.kcap = a.kcap; g.bs = a.bs;
     g.W = a.window; g.token_cutoff = 1; g.scale = a.scale;
-    if (a.mode == kSwa) launch_page_attn<kPageSwa>(g, a.d, stream);
+    if (a.mode == kSwa && win_path(a.window, 0, a.scale, 0, a.tq, 0) && win_fills(0, a.tq, a.batch, a.hq, a.hkv))
+      launch_win_attn<kPageSwa>(g, a.d, stream);
+    else if (a.mode == kSwa) launch_page_attn<kPageSwa>(g, a.d, stream);
     else if (a.mode == kHca) launch_page_attn<kPageDense>(g, a.d, stream);
     else launch_page_attn<kPageRouted>(g, a.d, stream);
     BFLY_CHECK_LAUNCH(what);

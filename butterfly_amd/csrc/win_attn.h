@@ -1,0 +1,421 @@
+// bf16 window + summary attention for windows of up to 128 tokens with every key of a unit in one
+// softmax (head_dim 64, 128 or 256): what the windows of 65..128 tokens run on.
+//
+// Semantics and work unit as page_attn.h: (batch, kv head, HW * NH of its query heads, 64 consecutive
+// query positions).  The unit's keys are 192 window rows (positions 64 c - 128 .. 64 c + 63) and a
+// 16-slot tile of routed summaries.  Two phases share one LDS buffer of 208 rows:
+//   * K staged; each wave (16 query rows, HW heads) scores its nine window tiles and the summary tile
+//     (S^T = K Q^T, one K fragment read for the wave's heads), one maximum and one sum per row in fp32
+//     registers, P = hi + lo in two bf16 parts;
+//   * V, requested with K and held in registers until every wave is done with K, staged in the same
+//     rows; O^T = V^T P^T tile by tile (one V fragment read for HW heads times two parts), stored as
+//     each 64 columns are done.
+// No running softmax: one maximum per row and chunk, no rescaling, and no output accumulators held
+// across the keys (page_attn_kernel holds D / 4 registers a head and runs 7 barriers a unit; 3 here).
+// The buffer is 110 KB at d = 256 (one workgroup of 512 threads per CU), 57 KB at d = 128 and 29 KB at
+// d = 64 (workgroups of 256 threads and two heads, two per CU by registers).
+//
+// An infinity or NaN in V: its rows are flagged when V is staged; a unit with any takes fragments with
+// such elements zeroed and adds them afterwards to the rows that attend to them.
+#pragma once
+
+#include "page_attn.h"
+
+namespace bfly {
+
+constexpr int kWinMax = 128;                  // window
+constexpr int kWinRows = 192;                 // staged window rows
+constexpr int kWinSlots = 16;                 // summary slots
+constexpr int kWinAll = kWinRows + kWinSlots;
+
+template <int D, int HW, int NH, int MODE, bool kBatch = false>
+__global__ void __launch_bounds__(256 * NH, 2)
+win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch> cb) {
+  PageArgs a = a_in;
+  constexpr int NTHR = 256 * NH, KP = D + 8, KSTEPS = D / 32, PIECES = D / 8, MT = D / 32;
+  constexpr int RSTEP = NTHR / PIECES;                       // rows between a thread's pieces
+  constexpr int LD = (kWinAll + RSTEP - 1) / RSTEP;          // K (and V) pieces per thread
+  constexpr int NT = MODE == kPageSwa ? 9 : 10;              // key tiles of a wave: 9 window, the summaries
+  static_assert(MODE == kPageFused || MODE == kPageSwa, "window modes");
+  static_assert(!kBatch || MODE == kPageFused, "batches are the streaming loop's");
+  static_assert(64 % RSTEP == 0 || RSTEP % 64 == 0, "a round of pieces lies in one page");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kWinAll * KP * 2];
+  __shared__ int s_n[kWinSlots], s_b[kWinSlots];
+  __shared__ int s_bad[kWinAll + 1];                         // rows of V with an infinity or NaN, and whether any
+  __bf16* Ks = reinterpret_cast<__bf16*>(smem);              // [kWinAll][KP], then V [kWinAll][D] swizzled
+  if constexpr (kBatch) {
+    static_assert(sizeof(smem) >= NH * 256 * 8 * 4, "pooling scratch aliases the staging rows");
+    if ((int)blockIdx.x >= cb.attn_blocks) {
+      page_update<NH>(cb, reinterpret_cast<float*>(smem));
+      return;
+    }
+  }
+  int row, chunk, zc;
+  if (!page_unit<kBatch>(a, cb, row, chunk, zc)) return;
+  const int bh = row / a.nparts, hpart = row - bh * a.nparts;
+  const int bi = bh / a.hkv, kvh = bh - bi * a.hkv;
+  const int gsz = a.hq / a.hkv;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int lg = lane >> 4, lq = lane & 15;
+  const int qwave = wave & 3;
+  const int h0 = (hpart * NH + (wave >> 2)) * HW;      // the wave's first head in the group
+
+  const int pw = chunk * kPageRows + qwave * 16;
+  const int qp = pw + lq;                               // this lane's query position (column lq)
+  const bool row_ok = qp >= a.qlo && qp < a.qhi;
+  const bool wave_on = pw + 15 >= a.qlo && pw < a.qhi && h0 < gsz;
+  auto blk_of = [&](int p) { return min(max(p / a.bs, 0), a.nblocks - 1); };
+  const int qblk = MODE == kPageSwa ? 0 : blk_of(qp);
+  const float sl2 = a.scale * 1.4426950408889634f;      // > 0 (the host's rule)
+
+  // ---- requests: Q, then every K row, then every V row
+  bf16x8 qf[HW][KSTEPS];
+  const int64_t qhead0 = ((int64_t)bi * a.hq + (int64_t)kvh * gsz) * a.tq;
+  const int qrow = row_ok ? qp - a.qlo : 0;
+#pragma unroll
+  for (int u = 0; u < HW; ++u) {
+    const __bf16* qs = reinterpret_cast<const __bf16*>(a.q) +
+                       (qhead0 + (int64_t)min(h0 + u, gsz - 1) * a.tq + qrow) * D + lg * (D / 4);
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) qf[u][ks] = *reinterpret_cast<const bf16x8*>(qs + 8 * ks);
+  }
+  const int p_lo = chunk * kPageRows - 128;             // position of LDS row 0
+  const int first = max(max(max(chunk * kPageRows, a.qlo) - a.W + 1, a.key_lo), 0);   // first key anyone needs
+  const int last = a.kv_len - 1;
+  const __bf16* kb = reinterpret_cast<const __bf16*>(a.k) + (int64_t)bh * a.kv_rows * D;
+  const __bf16* vb = reinterpret_cast<const __bf16*>(a.v) + (int64_t)bh * a.kv_rows * D;
+  page_u32x4 kst[LD], vst[LD];
+  // thread: piece pc of rows r0, r0 + RSTEP, ...  A row that no query of the unit attends to is read as
+  // the nearest one that exists (masked; its values are finite or flagged like any other)
+  const int pc = tid % PIECES, r0 = tid / PIECES;
+  const __bf16* kr[LD];
+  const __bf16* vr[LD];
+  const int p_min = min(first, last), p_base = max(p_lo, p_min);       // the lowest row read, >= key_lo or p_lo
+  const int base = a.ring ? (int)((unsigned)p_base % (unsigned)a.ring) : p_base - a.key_lo;
+#pragma unroll
+  for (int j = 0; j < LD; ++j) {
+    const int r = r0 + j * RSTEP;
+    if ((j + 1) * RSTEP <= kWinRows) {                  // (RSTEP divides 64: whole rounds of window rows)
+      const int p = min(max(p_lo + r, p_min), last);    // p_base <= p < p_base + kWinRows
+      const __bf16 *kx = kb, *vx = vb;
+      int x = base + (p - p_base);
+      if (a.ring && x >= a.ring) x -= a.ring;           // (the host: ring >= kWinRows)
+      if constexpr (kBatch) {
+        // the round's page; a row clamped below it (to `first`) or above it (to `last`) stays in the
+        // page's chunk or, below the batch, in the ring
+        const int pg = p_lo + (j * RSTEP) / kPageRows * kPageRows;
+        if (cb.from_inputs && pg >= cb.c[0].qlo) {
+          const void *kc, *vc;
+          int lo, len;
+          page_input(cb, pg, kc, vc, lo, len);
+          kx = reinterpret_cast<const __bf16*>(kc) + (int64_t)bh * len * D;
+          vx = reinterpret_cast<const __bf16*>(vc) + (int64_t)bh * len * D;
+          x = min(max(p - lo, 0), len - 1);
+        } else if (cb.from_inputs) {
+          // a page before the batch: rows clamped up into the batch read its first ring row instead
+          x = p < cb.c[0].qlo ? x : 0;
+        }
+      }
+      kr[j] = kx + (int64_t)x * D + pc * 8;
+      vr[j] = vx + (int64_t)x * D + pc * 8;
+    } else {
+      kr[j] = kb;
+      vr[j] = vb;
+    }
+  }
+  const int q_first = max(chunk * kPageRows, a.qlo), q_last = min((chunk + 1) * kPageRows, a.qhi) - 1;
+  const int bA = MODE == kPageSwa ? 0 : blk_of(q_first), bB = MODE == kPageSwa ? 0 : blk_of(q_last);
+  for (int i = tid; i < kWinAll + 1; i += NTHR) s_bad[i] = 0;
+  if constexpr (MODE == kPageFused) page_slots<kBatch>(a, cb, zc, bA, bB, kWinSlots, s_n, s_b);
+#pragma unroll
+  for (int j = 0; j < LD; ++j)
+    if ((j + 1) * RSTEP <= kWinRows) kst[j] = *reinterpret_cast<const page_u32x4*>(kr[j]);
+  __syncthreads();   // the summary slots
+  if constexpr (MODE == kPageFused) {
+    // (without summaries their tile is masked and its rows are window row 0's)
+    const __bf16* ks = a.nsum > 0 ? reinterpret_cast<const __bf16*>(a.ks) + (int64_t)bh * a.pool_rows * D : kb;
+    const __bf16* vs = a.nsum > 0 ? reinterpret_cast<const __bf16*>(a.vs) + (int64_t)bh * a.pool_rows * D : vb;
+#pragma unroll
+    for (int j = 0; j < LD; ++j)
+      if ((j + 1) * RSTEP > kWinRows) {
+        const int64_t n = max(s_n[(r0 + j * RSTEP - kWinRows) & (kWinSlots - 1)], 0);
+        kr[j] = ks + n * D + pc * 8;
+        vr[j] = vs + n * D + pc * 8;
+        kst[j] = *reinterpret_cast<const page_u32x4*>(kr[j]);
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < LD; ++j)
+    if ((j + 1) * RSTEP <= kWinRows || MODE == kPageFused) vst[j] = *reinterpret_cast<const page_u32x4*>(vr[j]);
+  // rows staged (the last round of d = 64 runs past the summary slots)
+  auto staged = [&](int j) { return (j + 1) * RSTEP <= kWinRows || (MODE == kPageFused && r0 + j * RSTEP < kWinAll); };
+#pragma unroll
+  for (int j = 0; j < LD; ++j)
+    if (staged(j)) *reinterpret_cast<page_u32x4*>(Ks + (r0 + j * RSTEP) * KP + pc * 8) = kst[j];
+  __syncthreads();   // K staged
+
+  // ---- scores and softmax: key 4 lg + i of tile t (window tiles: positions pw - 128 + 16 t .., rows
+  // 16 (qwave + t) ..; tile 9: the summary slots)
+  bf16x8 hi[HW][5], lo[HW][5];
+  float inv[HW];
+  const int wlo = max(max(qp - a.W + 1, a.key_lo), 0);
+  const int qcut = max(0, (a.token_cutoff ? qp : qblk * a.bs) - a.W + 1);
+  auto sum_ok = [&](int s) {
+    const int n = s_n[s];
+    return n >= 0 && s_b[s] == qblk && (n + 1) * a.bs <= qcut;
+  };
+  if (wave_on) {
+    f32x4 s[HW][10];
+    const __bf16* kl = Ks + (16 * qwave + lq) * KP + lg * (D / 4);
+    const __bf16* kq = Ks + (kWinRows + lq) * KP + lg * (D / 4);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      bf16x8 kf[KSTEPS];
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+        kf[ks] = *reinterpret_cast<const bf16x8*>((t < 9 ? kl + 16 * t * KP : kq) + 8 * ks);
+#pragma unroll
+      for (int u = 0; u < HW; ++u) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], qf[u][ks], acc, 0, 0, 0);
+        s[u][t] = acc;
+      }
+    }
+    // window keys [wlo, qp] as offsets from this lane group's first key of tile 0
+    const int off = pw - 128 + 4 * lg, klo = wlo - off, khi = min(qp, last) - off;
+#pragma unroll
+    for (int t = 0; t < 10; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bool ok;
+        if (t < 8) ok = 16 * t + i >= klo;              // (before pw: not above the query)
+        else if (t == 8) ok = 128 + i >= klo && 128 + i <= khi;
+        else ok = MODE == kPageFused && sum_ok(4 * lg + i);
+#pragma unroll
+        for (int u = 0; u < HW; ++u) {
+          if (t < NT) s[u][t][i] = ok ? s[u][t][i] : -INFINITY;
+          else s[u][t][i] = -INFINITY;
+        }
+      }
+#pragma unroll
+    for (int u = 0; u < HW; ++u) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) mx = fmaxf(mx, fmaxf(fmaxf(s[u][t][0], s[u][t][1]), fmaxf(s[u][t][2], s[u][t][3])));
+      mx = col_max4(mx);
+      const float nm = mx == -INFINITY ? 0.f : -mx * sl2;
+      float l = 0.f;
+#pragma unroll
+      for (int t = 0; t < 10; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float e = 0.f;
+          if (t < NT) {
+            e = __builtin_amdgcn_exp2f(fmaf(s[u][t][i], sl2, nm));
+            l += e;
+          }
+          const __bf16 h = (__bf16)e;
+          hi[u][t / 2][(t % 2) * 4 + i] = h;
+          lo[u][t / 2][(t % 2) * 4 + i] = (__bf16)(e - (float)h);
+        }
+      l = col_sum4(l);
+      if constexpr (MODE == kPageFused) {
+        inv[u] = 1.f / fmaxf(l, 1e-30f);
+        // every window score -inf (or NaN): 0 / 0, as one softmax over the row's keys gives
+        if (mx == -INFINITY && wlo <= min(qp, last)) inv[u] = NAN;
+      } else {
+        const bool any = mx != -INFINITY;
+        inv[u] = any ? 1.f / l : 0.f;
+        if (lg == 0 && row_ok && h0 + u < gsz) {
+          const int64_t r = qhead0 + (int64_t)(h0 + u) * a.tq + (qp - a.qlo);
+          a.l[r] = any ? l : 0.f;
+          a.m[r] = any ? mx * a.scale : kPageNeg;
+        }
+      }
+    }
+  }
+  __syncthreads();   // every wave is done with K
+  __bf16* Vs = Ks;
+#pragma unroll
+  for (int j = 0; j < LD; ++j)
+    if (staged(j)) {
+      const int r = r0 + j * RSTEP;
+      *reinterpret_cast<page_u32x4*>(Vs + r * D + (pc ^ vrow_swizzle<D>(r)) * 8) = vst[j];
+      if (page_nonfinite(vst[j])) s_bad[r] = s_bad[kWinAll] = 1;
+    }
+  __syncthreads();   // V staged
+  if (!wave_on) return;
+  const bool bad = s_bad[kWinAll] != 0;
+
+  // ---- O^T = V^T P^T.  V fragments (transposing reads): row 4 lg + (lq >> 2) of a tile, 8-byte unit
+  // mt * 8 + (lq & 3) * 2 + half XOR the row's swizzle, which is this lane's alone
+  const int xs = D == 64 ? (lq >> 3) & 1 : (lq >> 2) & 3;
+  const __bf16* vrow = Vs + (4 * lg + (lq >> 2)) * D;
+  const int vcol = (lq & 3) * 8;
+  const bool lo8 = lq < 8;
+  const int pA = pw + (lq & 7), pB = pA + 8;
+  const bool okA = pA >= a.qlo && pA < a.qhi, okB = pB >= a.qlo && pB < a.qhi;
+  __bf16* ob = reinterpret_cast<__bf16*>(a.out) + (qhead0 + (int64_t)h0 * a.tq) * D;
+  const int64_t hstride = (int64_t)a.tq * D;
+  const int64_t oA = (int64_t)(okA ? pA - a.qlo : 0) * D, oB = (int64_t)(okB ? pB - a.qlo : 0) * D;
+  auto finite = [](bf16x4 x) {      // infinities and NaN as zeros
+    typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+    u16x4 b = __builtin_bit_cast(u16x4, x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = (b[e] & 0x7f80) == 0x7f80 ? 0 : b[e];
+    return __builtin_bit_cast(bf16x4, b);
+  };
+  // output tiles mt = 2 mp, 2 mp + 1: one 128-byte line per position
+  auto columns = [&](int mp, auto has_bad) {
+    constexpr bool kBad = decltype(has_bad)::value;
+    bf16x8 w[HW][2];
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      const int mt = 2 * mp + sub;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        f32x4 o[HW];
+#pragma unroll
+        for (int u = 0; u < HW; ++u) o[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const __bf16* vp = vrow + (mt ^ xs) * 32 + vcol + half * 4;
+#pragma unroll
+        for (int pr = 0; pr < 5; ++pr) {
+          bf16x4 va = read_tr(vp + 16 * (qwave + 2 * pr) * D);
+          bf16x4 vc = {};
+          if (pr < 4) vc = read_tr(vp + 16 * (qwave + 2 * pr + 1) * D);
+          else if (MODE == kPageFused) vc = read_tr(vp + kWinRows * D);
+          if constexpr (kBad) {
+            va = finite(va);
+            vc = finite(vc);
+          }
+          const bf16x8 vf = __builtin_shufflevector(va, vc, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+          for (int u = 0; u < HW; ++u) {
+            o[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi[u][pr], o[u], 0, 0, 0);
+            o[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo[u][pr], o[u], 0, 0, 0);
+          }
+        }
+        if constexpr (kBad) {
+          // flagged rows one by one: this lane's 4 d of the rows that its query attends to
+#pragma unroll 1
+          for (int r = 0; r < kWinAll; ++r) {
+            if (!s_bad[r]) continue;
+            const int rel = r < kWinRows ? r - 16 * qwave : 144 + r - kWinRows;   // row of the wave's ten tiles
+            if (rel < 0 || (r < kWinRows && rel >= 144)) continue;
+            const bool take = r < kWinRows ? p_lo + r >= wlo && p_lo + r <= min(qp, last) : sum_ok(r - kWinRows);
+            const int src = lq + 16 * ((rel >> 2) & 3), pick = (rel >> 4) * 4 + (rel & 3);
+            const int unit = mt * 8 + lg * 2 + half;
+            const bf16x4 x = *reinterpret_cast<const bf16x4*>(Vs + r * D + (unit ^ (2 * vrow_swizzle<D>(r))) * 4);
+#pragma unroll
+            for (int u = 0; u < HW; ++u) {
+              float p = 0.f;
+#pragma unroll
+              for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                  p = pick == 4 * t + i ? (float)hi[u][t / 2][(t % 2) * 4 + i] + (float)lo[u][t / 2][(t % 2) * 4 + i] : p;
+              p = __shfl(p, src);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float xv = (float)x[e];
+                if (take && !(fabsf(xv) < INFINITY)) o[u][e] = fmaf(p, xv, o[u][e]);
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < HW; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w[u][sub][4 * half + i] = (__bf16)(o[u][i] * inv[u]);
+      }
+    }
+    // lanes lq and lq ^ 8 swap a 16-byte piece so that each store writes 8 whole lines
+    const int dA = (2 * mp + (lo8 ? 0 : 1)) * 32 + lg * 8;
+#pragma unroll
+    for (int u = 0; u < HW; ++u) {
+      if (h0 + u >= gsz) continue;
+      const bf16x8 x = page_xchg8(lo8 ? w[u][1] : w[u][0]);
+      const bf16x8 sa = lo8 ? w[u][0] : x, sb = lo8 ? x : w[u][1];
+      if (okA) __builtin_nontemporal_store(sa, reinterpret_cast<bf16x8*>(ob + u * hstride + oA + dA));
+      if (okB) __builtin_nontemporal_store(sb, reinterpret_cast<bf16x8*>(ob + u * hstride + oB + dA));
+    }
+  };
+  if (!bad) {
+#pragma unroll
+    for (int mp = 0; mp < MT / 2; ++mp) columns(mp, std::false_type{});
+  } else {
+#pragma unroll 1
+    for (int mp = 0; mp < MT / 2; ++mp) columns(mp, std::true_type{});
+  }
+}
+
+// Whether win_attn_kernel takes a launch that page_attn_kernel takes: 64 < W <= 128 (a shorter window
+// wastes most of its nine tiles), summaries in one tile, rows to stand in for those that do not
+// exist, a ring that the staged rows do not wrap twice.
+static inline bool win_path(int64_t W, int64_t slots, float scale, int64_t key_lo, int64_t kv_len, int64_t ring) {
+  return W > 64 && W <= kWinMax && slots <= kWinSlots && scale > 0.f && key_lo < kv_len && (ring == 0 || ring >= kWinRows);
+}
+
+// Whether the grid fills the chip with the split that launch_win_attn takes (two heads per workgroup, or
+// the group's one).  Smaller launches leave most CUs idle either way and page_attn_kernel, which starts
+// on its first 64 keys, ends sooner: 512 rows over a 32k plain cache, 16/4 heads of d 128, 28.6 us with
+// the compressor against 32.4.
+static inline bool win_fills(int64_t qlo, int64_t tq, int64_t batch, int hq, int hkv) {
+  const int64_t chunks = (qlo + tq - 1) / kPageRows - qlo / kPageRows + 1;
+  const int gsz = hq / hkv;
+  return chunks * batch * hkv * (gsz > 1 ? (gsz + 1) / 2 : 1) >= 256;
+}
+
+template <int MODE>
+static inline void launch_win_attn(PageArgs a, int d, hipStream_t stream) {
+  a.c_first = a.qlo / kPageRows;
+  a.nchunks = (a.qhi - 1) / kPageRows - a.c_first + 1;
+  const int gsz = a.hq / a.hkv;
+  const int64_t units = (int64_t)a.nchunks * a.batch * a.hkv;
+  auto go = [&](auto kernel, int heads, int nh) {
+    a.nparts = (gsz + heads - 1) / heads;
+    a.items = (int)(units * a.nparts);
+    a.per_xcd = (a.items + 7) / 8;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * a.per_xcd)), dim3(256 * nh), 0, stream, a, PageNoBatch{});
+  };
+  const bool two = gsz >= 2;
+  if (d == 256) {
+    if (gsz >= 3 && units * ((gsz + 3) / 4) >= 256) go(win_attn_kernel<256, 2, 2, MODE>, 4, 2);
+    else go(win_attn_kernel<256, 1, 2, MODE>, 2, 2);
+  } else if (d == 128) {
+    if (two) go(win_attn_kernel<128, 2, 1, MODE>, 2, 1);
+    else go(win_attn_kernel<128, 1, 1, MODE>, 1, 1);
+  } else {
+    if (two) go(win_attn_kernel<64, 2, 1, MODE>, 2, 1);
+    else go(win_attn_kernel<64, 1, 1, MODE>, 1, 1);
+  }
+}
+
+// launch_page_batch on win_attn_kernel.
+static inline void launch_win_batch(PageArgs a, PageBatch cb, int d, int nchunks_max, hipStream_t stream) {
+  const int gsz = a.hq / a.hkv;
+  auto go = [&](auto kernel, int heads, int nh) {
+    a.c_first = 0;
+    a.nchunks = nchunks_max;
+    a.nparts = (gsz + heads - 1) / heads;
+    a.items = nchunks_max * cb.nch * a.batch * a.hkv * a.nparts;
+    a.per_xcd = (a.items + 7) / 8;
+    cb.attn_blocks = 8 * a.per_xcd;
+    const int64_t extra = (cb.upd_wgs + nh - 1) / nh;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(cb.attn_blocks + extra)), dim3(256 * nh), 0, stream, a, cb);
+  };
+  const int64_t units = (int64_t)nchunks_max * cb.nch * a.batch * a.hkv;
+  if (d == 256) {
+    if (gsz >= 3 && units * ((gsz + 3) / 4) >= 128) go(win_attn_kernel<256, 2, 2, kPageFused, true>, 4, 2);
+    else go(win_attn_kernel<256, 1, 2, kPageFused, true>, 2, 2);
+  } else if (d == 128) {
+    if (gsz > 1) go(win_attn_kernel<128, 2, 1, kPageFused, true>, 2, 1);
+    else go(win_attn_kernel<128, 1, 1, kPageFused, true>, 1, 1);
+  } else {
+    if (gsz > 1) go(win_attn_kernel<64, 2, 1, kPageFused, true>, 2, 1);
+    else go(win_attn_kernel<64, 1, 1, kPageFused, true>, 1, 1);
+  }
+}
+
+}  // namespace bfly

@@ -1,7 +1,7 @@
 """GPU: the paged MFMA kernel (windows above 64, blocks below 64, the bf16 streams) against the oracle.
 
 The oracle runs in float32 over the same bf16 inputs and the device's own bf16 summaries, so what
-remains is the output's rounding to bf16 (half an ulp, at most 2^-9 of the value) and fp32
+remains is the output's rounding to bf16 (half an ulp, at most 2^-8 of the value) and fp32
 arithmetic: scores and weights carry a relative error of about 1e-6, times values of up to 5.
 """
 from __future__ import annotations
@@ -226,7 +226,8 @@ STREAMS = [
 @pytest.mark.parametrize("case", STREAMS, ids=lambda c: "-".join(str(x) for x in c[:7]))
 def test_stream_batches_match_single_chunks(case):
     """chunked_prefill (batched launches, updates beside attention) against one core call per chunk:
-    outputs, tail, pools and counters bit for bit."""
+    tail, pools and counters bit for bit, and the outputs too -- up to each side's own rounding to bf16
+    (2^-8 of the value and ABS) at W 65..128, where single chunks and batches may take two kernels."""
     d, hq, hkv, w, cw, bs, max_chunk, lens = case
     cfg = bf.compressed_butterfly_config(block_size=bs, compressed_local_window_tokens=w, block_partner_rule="xor")
     g = torch.Generator(device="cuda").manual_seed(5)
@@ -238,7 +239,10 @@ def test_stream_batches_match_single_chunks(case):
     assert core.last_profile.notes.get("native_chunk_loop")
     want = [core(*c, caches[1]) for c in chunks]
     for i, (a, b) in enumerate(zip(got, want)):
-        assert torch.equal(a, b), i
+        if 64 < w <= 128:
+            assert ((a.float() - b.float()).abs() <= 2 * BF16_ROUNDING * b.float().abs() + 2 * ABS).all(), i
+        else:
+            assert torch.equal(a, b), i
     x, y = caches
     assert (x.offset, x.tail_size, x.summary_count, x.summary_offset) == \
         (y.offset, y.tail_size, y.summary_count, y.summary_offset)

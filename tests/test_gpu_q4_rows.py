@@ -1,6 +1,6 @@
 """GPU: products of 2 to 32 rows from the 4-bit codes (bfly_q4_rows, bfly_q4_rows_silu).
 
-Against 64-bit sums over w = code * scale + bias: the output's rounding to bf16 (2^-9 of the value),
+Against 64-bit sums over w = code * scale + bias: the output's rounding to bf16 (at most 2^-8 of the value),
 and fp32 sums of terms x (16 + code) scale and x (bias - 16 scale), whose error is below
 2^-20 of the sum of their magnitudes (four roundings of 2^-24 on each, few-fold accumulation).
 """

@@ -1470,7 +1470,7 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
       default: hipLaunchKernelGGL(attn_mfma_kernel<256>, grid, dim3(MfmaCfg<256>::NTHR), 0, stream, a, m, seg, (int)c_first, (int)nchunks, hper, NoBatch{}); break;
     }
   } else if (dtype == BFLY_DTYPE_BF16 && contiguous && page_path(a, chunk_blocks_max(a.bs))) {
-    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, a.key_lo, a.kv_len, a.ring) &&
+    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, a.key_lo, a.kv_len) &&
         win_fills(a.q_pos0, a.tq, a.batch, a.hq, a.hkv))
       launch_win_attn<kPageFused>(page_args(a), a.d, stream);
     else
@@ -1564,7 +1564,7 @@ static int launch_attention_batch(const AttnArgs* ch, const void* const* kin, co
       pb.upd_wgs = ux * upd_rows * 2;
     }
     BFLY_CHECK_ARG(nch_max * n * groups * (a.hq / a.hkv) + pb.upd_wgs < (1 << 30), "%s: grid too large", what);
-    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, 0, 1, a.ring))
+    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, 0, 1))
       launch_win_batch(page_args(a), pb, a.d, (int)nch_max, stream);
     else
       launch_page_batch(page_args(a), pb, a.d, (int)nch_max, stream);

@@ -228,7 +228,7 @@ static int launch_stream(const StreamArgs& a, int dtype, hipStream_t stream, con
     g.qlo = 0; g.qhi = (int)a.tq; g.key_lo = 0; g.kv_len = (int)a.tq; g.ring = 0;
     g.nblocks = (int)((a.tq + a.bs - 1) / a.bs); g.nsum = (int)a.nsum; g.kcap = a.kcap; g.bs = a.bs;
     g.W = a.window; g.token_cutoff = 1; g.scale = a.scale;
-    if (a.mode == kSwa && win_path(a.window, 0, a.scale, 0, a.tq, 0) && win_fills(0, a.tq, a.batch, a.hq, a.hkv))
+    if (a.mode == kSwa && win_path(a.window, 0, a.scale, 0, a.tq) && win_fills(0, a.tq, a.batch, a.hq, a.hkv))
       launch_win_attn<kPageSwa>(g, a.d, stream);
     else if (a.mode == kSwa) launch_page_attn<kPageSwa>(g, a.d, stream);
     else if (a.mode == kHca) launch_page_attn<kPageDense>(g, a.d, stream);

@@ -28,6 +28,22 @@ constexpr int kWinRows = 192;                 // staged window rows
 constexpr int kWinSlots = 16;                 // summary slots
 constexpr int kWinAll = kWinRows + kWinSlots;
 
+// max(a, b, c) in one instruction (fmaxf first quiets each operand that may be a signalling NaN)
+__device__ __forceinline__ float win_max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// The larger of `m`'s halves and those of a piece's bf16 without their signs, half by half.
+__device__ __forceinline__ unsigned win_magnitude(unsigned m, page_u32x4 x) {
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 r = __builtin_bit_cast(u16x2, m);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r = __builtin_elementwise_max(r, __builtin_bit_cast(u16x2, x[i] & 0x7fff7fffu));
+  return __builtin_bit_cast(unsigned, r);
+}
+
 template <int D, int HW, int NH, int MODE, bool kBatch = false>
 __global__ void __launch_bounds__(256 * NH, 2)
 win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch> cb) {
@@ -38,7 +54,8 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
   constexpr int NT = MODE == kPageSwa ? 9 : 10;              // key tiles of a wave: 9 window, the summaries
   static_assert(MODE == kPageFused || MODE == kPageSwa, "window modes");
   static_assert(!kBatch || MODE == kPageFused, "batches are the streaming loop's");
-  static_assert(64 % RSTEP == 0 || RSTEP % 64 == 0, "a round of pieces lies in one page");
+  static_assert(64 % RSTEP == 0 && RSTEP >= kWinSlots && LD * RSTEP >= kWinAll && (LD - 1) * RSTEP == kWinRows,
+                "a round of pieces lies in one page, the summary slots in the last");
   __shared__ __attribute__((aligned(16))) unsigned char smem[kWinAll * KP * 2];
   __shared__ int s_n[kWinSlots], s_b[kWinSlots];
   __shared__ int s_bad[kWinAll + 1];                         // rows of V with an infinity or NaN, and whether any
@@ -80,73 +97,96 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
     for (int ks = 0; ks < KSTEPS; ++ks) qf[u][ks] = *reinterpret_cast<const bf16x8*>(qs + 8 * ks);
   }
   const int p_lo = chunk * kPageRows - 128;             // position of LDS row 0
-  const int first = max(max(max(chunk * kPageRows, a.qlo) - a.W + 1, a.key_lo), 0);   // first key anyone needs
-  const int last = a.kv_len - 1;
+  const int last = a.kv_len - 1, key0 = max(a.key_lo, 0);
   const __bf16* kb = reinterpret_cast<const __bf16*>(a.k) + (int64_t)bh * a.kv_rows * D;
   const __bf16* vb = reinterpret_cast<const __bf16*>(a.v) + (int64_t)bh * a.kv_rows * D;
   page_u32x4 kst[LD], vst[LD];
-  // thread: piece pc of rows r0, r0 + RSTEP, ...  A row that no query of the unit attends to is read as
-  // the nearest one that exists (masked; its values are finite or flagged like any other)
+  // thread: piece pc of rows r0, r0 + RSTEP, ...; the window rows are three pages of 64
+  constexpr int RPP = 64 / RSTEP;                       // rounds per page
   const int pc = tid % PIECES, r0 = tid / PIECES;
-  const __bf16* kr[LD];
-  const __bf16* vr[LD];
-  const int p_min = min(first, last), p_base = max(p_lo, p_min);       // the lowest row read, >= key_lo or p_lo
-  const int base = a.ring ? (int)((unsigned)p_base % (unsigned)a.ring) : p_base - a.key_lo;
+  const unsigned voff = (unsigned)(r0 * D + pc * 8);
+  // Page g's rows, K or V (kv): a page whose 64 positions all exist and lie in one run of rows is read at
+  // uniform addresses plus voff.  In any other, a position that does not exist reads the nearest one
+  // that does (masked; its V is finite or flagged like any other), each row found by itself.
+  struct Run {
+    const __bf16 *k, *v;
+    bool whole;
+  } run[3];
 #pragma unroll
-  for (int j = 0; j < LD; ++j) {
-    const int r = r0 + j * RSTEP;
-    if ((j + 1) * RSTEP <= kWinRows) {                  // (RSTEP divides 64: whole rounds of window rows)
-      const int p = min(max(p_lo + r, p_min), last);    // p_base <= p < p_base + kWinRows
-      const __bf16 *kx = kb, *vx = vb;
-      int x = base + (p - p_base);
-      if (a.ring && x >= a.ring) x -= a.ring;           // (the host: ring >= kWinRows)
-      if constexpr (kBatch) {
-        // the round's page; a row clamped below it (to `first`) or above it (to `last`) stays in the
-        // page's chunk or, below the batch, in the ring
-        const int pg = p_lo + (j * RSTEP) / kPageRows * kPageRows;
-        if (cb.from_inputs && pg >= cb.c[0].qlo) {
-          const void *kc, *vc;
-          int lo, len;
-          page_input(cb, pg, kc, vc, lo, len);
-          kx = reinterpret_cast<const __bf16*>(kc) + (int64_t)bh * len * D;
-          vx = reinterpret_cast<const __bf16*>(vc) + (int64_t)bh * len * D;
-          x = min(max(p - lo, 0), len - 1);
-        } else if (cb.from_inputs) {
-          // a page before the batch: rows clamped up into the batch read its first ring row instead
-          x = p < cb.c[0].qlo ? x : 0;
+  for (int g = 0; g < 3; ++g) {
+    const int p0 = p_lo + 64 * g;
+    const __bf16 *kx = kb, *vx = vb;
+    int x = p0 - a.key_lo;
+    bool whole = p0 >= key0 && p0 + 63 <= last;
+    bool ring = a.ring != 0;
+    if constexpr (kBatch) {
+      if (cb.from_inputs && p0 >= cb.c[0].qlo) {
+        // the chunk of the batch that holds the page: this one or one before it
+        int zp = zc;
+        while (zp > 0 && p0 < cb.c[zp].qlo) --zp;
+        const int len = cb.c[zp].tq;
+        kx = reinterpret_cast<const __bf16*>(cb.c[zp].k) + (int64_t)bh * len * D;
+        vx = reinterpret_cast<const __bf16*>(cb.c[zp].v) + (int64_t)bh * len * D;
+        x = p0 - cb.c[zp].qlo;
+        ring = false;
+      }
+    }
+    if (ring && whole) {
+      x = (int)((unsigned)p0 % (unsigned)a.ring);
+      whole = x + 64 <= a.ring;
+    }
+    run[g].k = whole ? kx + (int64_t)x * D : kx;
+    run[g].v = whole ? vx + (int64_t)x * D : vx;
+    run[g].whole = whole;
+  }
+  auto load_pages = [&](int kv, page_u32x4 (&dst)[LD]) {
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      const __bf16* src = kv ? run[g].v : run[g].k;
+      if (run[g].whole) {
+#pragma unroll
+        for (int i = 0; i < RPP; ++i)
+          dst[g * RPP + i] = *reinterpret_cast<const page_u32x4*>(src + (unsigned)(i * RSTEP * D) + voff);
+      } else {
+        const int p0 = p_lo + 64 * g;
+        int lo = key0, hi = last, first = a.key_lo, ring = a.ring;
+        if constexpr (kBatch) {
+          if (cb.from_inputs) {
+            if (p0 >= cb.c[0].qlo) {                    // (its chunk ends in the page or past it)
+              int zp = zc;
+              while (zp > 0 && p0 < cb.c[zp].qlo) --zp;
+              first = lo = cb.c[zp].qlo;
+              hi = min(last, lo + cb.c[zp].tq - 1);
+              ring = 0;
+            } else {
+              hi = cb.c[0].qlo - 1;                     // the batch's own tokens need not be in the ring
+            }
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < RPP; ++i) {
+          const int p = min(max(p0 + i * RSTEP + r0, lo), hi);
+          const int64_t x = ring ? (int64_t)((unsigned)p % (unsigned)ring) : (int64_t)(p - first);
+          dst[g * RPP + i] = *reinterpret_cast<const page_u32x4*>(src + x * D + pc * 8);
         }
       }
-      kr[j] = kx + (int64_t)x * D + pc * 8;
-      vr[j] = vx + (int64_t)x * D + pc * 8;
-    } else {
-      kr[j] = kb;
-      vr[j] = vb;
     }
-  }
+  };
   const int q_first = max(chunk * kPageRows, a.qlo), q_last = min((chunk + 1) * kPageRows, a.qhi) - 1;
   const int bA = MODE == kPageSwa ? 0 : blk_of(q_first), bB = MODE == kPageSwa ? 0 : blk_of(q_last);
   for (int i = tid; i < kWinAll + 1; i += NTHR) s_bad[i] = 0;
+  load_pages(0, kst);
   if constexpr (MODE == kPageFused) page_slots<kBatch>(a, cb, zc, bA, bB, kWinSlots, s_n, s_b);
-#pragma unroll
-  for (int j = 0; j < LD; ++j)
-    if ((j + 1) * RSTEP <= kWinRows) kst[j] = *reinterpret_cast<const page_u32x4*>(kr[j]);
+  load_pages(1, vst);
   __syncthreads();   // the summary slots
   if constexpr (MODE == kPageFused) {
-    // (without summaries their tile is masked and its rows are window row 0's)
+    // (without summaries their tile is masked and its rows are the window buffer's first)
     const __bf16* ks = a.nsum > 0 ? reinterpret_cast<const __bf16*>(a.ks) + (int64_t)bh * a.pool_rows * D : kb;
     const __bf16* vs = a.nsum > 0 ? reinterpret_cast<const __bf16*>(a.vs) + (int64_t)bh * a.pool_rows * D : vb;
-#pragma unroll
-    for (int j = 0; j < LD; ++j)
-      if ((j + 1) * RSTEP > kWinRows) {
-        const int64_t n = max(s_n[(r0 + j * RSTEP - kWinRows) & (kWinSlots - 1)], 0);
-        kr[j] = ks + n * D + pc * 8;
-        vr[j] = vs + n * D + pc * 8;
-        kst[j] = *reinterpret_cast<const page_u32x4*>(kr[j]);
-      }
+    const int64_t off = (int64_t)max(s_n[r0 & (kWinSlots - 1)], 0) * D + pc * 8;
+    kst[LD - 1] = *reinterpret_cast<const page_u32x4*>(ks + off);
+    vst[LD - 1] = *reinterpret_cast<const page_u32x4*>(vs + off);
   }
-#pragma unroll
-  for (int j = 0; j < LD; ++j)
-    if ((j + 1) * RSTEP <= kWinRows || MODE == kPageFused) vst[j] = *reinterpret_cast<const page_u32x4*>(vr[j]);
   // rows staged (the last round of d = 64 runs past the summary slots)
   auto staged = [&](int j) { return (j + 1) * RSTEP <= kWinRows || (MODE == kPageFused && r0 + j * RSTEP < kWinAll); };
 #pragma unroll
@@ -182,27 +222,33 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
         s[u][t] = acc;
       }
     }
-    // window keys [wlo, qp] as offsets from this lane group's first key of tile 0
+    // window keys [wlo, qp] as offsets from this lane group's first key of tile 0; tiles before pw hold no
+    // key above the queries, and those from the 16 rows' highest lower end on need no mask
     const int off = pw - 128 + 4 * lg, klo = wlo - off, khi = min(qp, last) - off;
+    const int full = max(max(pw + 15 - a.W + 1, a.key_lo), 0) - (pw - 128);
 #pragma unroll
-    for (int t = 0; t < 10; ++t)
+    for (int t = 0; t < 8; ++t)
+      if (16 * t < full) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bool ok;
-        if (t < 8) ok = 16 * t + i >= klo;              // (before pw: not above the query)
-        else if (t == 8) ok = 128 + i >= klo && 128 + i <= khi;
-        else ok = MODE == kPageFused && sum_ok(4 * lg + i);
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int u = 0; u < HW; ++u) {
-          if (t < NT) s[u][t][i] = ok ? s[u][t][i] : -INFINITY;
-          else s[u][t][i] = -INFINITY;
-        }
+          for (int u = 0; u < HW; ++u) s[u][t][i] = 16 * t + i >= klo ? s[u][t][i] : -INFINITY;
       }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool own = 128 + i >= klo && 128 + i <= khi;
+      const bool sum = MODE == kPageFused && sum_ok(4 * lg + i);
+#pragma unroll
+      for (int u = 0; u < HW; ++u) {
+        s[u][8][i] = own ? s[u][8][i] : -INFINITY;
+        if (MODE == kPageFused) s[u][9][i] = sum ? s[u][9][i] : -INFINITY;
+      }
+    }
 #pragma unroll
     for (int u = 0; u < HW; ++u) {
       float mx = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) mx = fmaxf(mx, fmaxf(fmaxf(s[u][t][0], s[u][t][1]), fmaxf(s[u][t][2], s[u][t][3])));
+      for (int t = 0; t < NT; ++t) mx = win_max3(win_max3(mx, s[u][t][0], s[u][t][1]), s[u][t][2], s[u][t][3]);
       mx = col_max4(mx);
       const float nm = mx == -INFINITY ? 0.f : -mx * sl2;
       float l = 0.f;
@@ -237,13 +283,19 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
   }
   __syncthreads();   // every wave is done with K
   __bf16* Vs = Ks;
+  unsigned worst = 0;      // per half: the largest magnitude
 #pragma unroll
   for (int j = 0; j < LD; ++j)
     if (staged(j)) {
       const int r = r0 + j * RSTEP;
       *reinterpret_cast<page_u32x4*>(Vs + r * D + (pc ^ vrow_swizzle<D>(r)) * 8) = vst[j];
-      if (page_nonfinite(vst[j])) s_bad[r] = s_bad[kWinAll] = 1;
+      worst = win_magnitude(worst, vst[j]);
     }
+  if (max(worst << 16, worst & 0xffff0000u) >= 0x7f800000u) {
+#pragma unroll
+    for (int j = 0; j < LD; ++j)
+      if (staged(j) && page_nonfinite(vst[j])) s_bad[r0 + j * RSTEP] = s_bad[kWinAll] = 1;
+  }
   __syncthreads();   // V staged
   if (!wave_on) return;
   const bool bad = s_bad[kWinAll] != 0;
@@ -353,8 +405,8 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
 // Whether win_attn_kernel takes a launch that page_attn_kernel takes: 64 < W <= 128 (a shorter window
 // wastes most of its nine tiles), summaries in one tile, rows to stand in for those that do not
 // exist, a ring that the staged rows do not wrap twice.
-static inline bool win_path(int64_t W, int64_t slots, float scale, int64_t key_lo, int64_t kv_len, int64_t ring) {
-  return W > 64 && W <= kWinMax && slots <= kWinSlots && scale > 0.f && key_lo < kv_len && (ring == 0 || ring >= kWinRows);
+static inline bool win_path(int64_t W, int64_t slots, float scale, int64_t key_lo, int64_t kv_len) {
+  return W > 64 && W <= kWinMax && slots <= kWinSlots && scale > 0.f && key_lo < kv_len;
 }
 
 // Whether the grid fills the chip with the split that launch_win_attn takes (two heads per workgroup, or

@@ -70,6 +70,8 @@ SIGNATURES = {
                                   _vp, _i64, _vp, _int, _i64, _int, _int, _int, _int, _int, _int, _f32, _vp, _vp]),
     "bfly_decode": (_int, [_vp, _int, _i64, _int, _int, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp,
                            _i64, _i64, C.POINTER(Topology), _i64, _int, _int, _f32, _vp, _vp]),
+    "bfly_decode_wide": (_int, [_vp, _int, _i64, _int, _int, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp,
+                           _i64, _i64, C.POINTER(Topology), _i64, _int, _int, _f32, _vp, _vp]),
     "bfly_decode_state_words": (_i64, [_i64, _int]),
     "bfly_decode_step": (_int, [_vp, _int, _i64, _int, _int, _int, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp,
                                 _i64, _int, _int, _int, _int, _int, _int, _int, _f32, _vp, _vp]),

@@ -384,8 +384,11 @@ class CompressedKVCache:
         blocks that fit were pooled, as the reference does.
         """
         self.sync()
-        offset0 = self.offset
-        step, first_pos, first_slot, n_new, overflow = self._advance(keys, values)
+        self._append(keys, values, self.offset, *self._advance(keys, values))
+
+    def _append(self, keys: torch.Tensor, values: torch.Tensor, offset0: int, step: int, first_pos: int,
+                first_slot: int, n_new: int, overflow: bool) -> None:
+        """The launch and the rest of the bookkeeping of ``update`` after ``_advance``."""
         b, h, d = int(keys.shape[0]), int(keys.shape[1]), int(keys.shape[3])
         keys, values = _c(keys), _c(values)
         with _on(keys.device):
@@ -411,23 +414,36 @@ class CompressedKVCache:
         as one fused launch (append + attention; plus the block compressor on the
         steps that complete a block); longer steps append, then attend.
         """
-        from .attention import _attend, _require_cuda, _scale
+        from .attention import _attend, _require_cuda, _scale, decode_row_entry
 
         _require_cuda(q)
         self.sync()
         step = int(keys.shape[2])
         d = int(q.shape[3])
         w = int(local_window_tokens)
-        fused = (step == 1 and int(q.shape[2]) == 1 and q.dtype == keys.dtype and w <= 64
-                 and layout.neighbors.shape[1] <= 16
-                 and (d in (64, 128) or (d == 256 and q.dtype == torch.bfloat16)))
-        if not fused:
+        nb = layout.neighbors
+        entry = None
+        if step == 1 and int(q.shape[2]) == 1 and q.dtype == keys.dtype:
+            made = self._ring_k is not None
+            # above 64, the general path's fewer conditions: a first step (no buffers yet), other shapes than the
+            # keys' and a cache that pools the newest block go there
+            if w <= 64 or (made and self.local_window_tokens > 0 and q.shape[0] == keys.shape[0]
+                           and d == keys.shape[3] == values.shape[3]):
+                bufs = (self._ring_k, self._ring_v, self._pool_k, self._pool_v) if made else ()
+                entry = decode_row_entry((q, *bufs), rows=self.tail_capacity, ring_capacity=self.tail_capacity,
+                                         kv_len=self.offset + 1, pool_rows=self.summary_capacity,
+                                         num_blocks=nb.shape[0], block_size=layout.block_size, window=w,
+                                         row_slots=nb.shape[1], scale=_scale(scale, d))
+        if entry is None:
             self.update(keys, values)
             return _attend(_c(q), self._ring_k, self._ring_v, self._pool_k, self._pool_v, layout=layout,
                            q_pos0=self.offset - int(q.shape[2]), qpos_dev=None, ring_capacity=self.tail_capacity,
                            tail_start=self.offset - self.tail_size, kv_len=self.offset,
                            summary_count=self.summary_count, local_window_tokens=w, scale=scale)
+        offset0 = self.offset
         _, first_pos, first_slot, n_new, overflow = self._advance(keys, values)
+        if overflow and w > 64:      # the token is appended before the pool's overflow raises
+            self._append(keys, values, offset0, 1, first_pos, first_slot, n_new, overflow)
         keys, values, q = _c(keys), _c(values), _c(q)
         st = _stream(q)
         self._compress(first_pos, first_slot, n_new, overflow, st)
@@ -435,9 +451,8 @@ class CompressedKVCache:
         self._push()
         b, hq = int(q.shape[0]), int(q.shape[1])
         out = torch.empty_like(q)
-        nb = layout.neighbors
         with _on(q.device):
-            _native.call("bfly_decode", q.data_ptr(), _dtype_code(q), b, hq, int(keys.shape[1]), d,
+            _native.call(entry, q.data_ptr(), _dtype_code(q), b, hq, int(keys.shape[1]), d,
                          keys.data_ptr(), values.data_ptr(), self._ring_k.data_ptr(), self._ring_v.data_ptr(),
                          self.tail_capacity, self.offset - self.tail_size, self.offset, self._pool_k.data_ptr(),
                          self._pool_v.data_ptr(), self.summary_capacity, self.summary_count, layout.table.topology,

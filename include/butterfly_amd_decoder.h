@@ -45,6 +45,17 @@ int bfly_qk_norm_rope(const void* q, const void* k, const void* v, int64_t q_row
                       int head_dim, float eps, void* q_out, void* k_out, void* v_out, hipStream_t stream);
 
 /*
+ * Device: bfly_qk_norm_rope for one new position per sequence that lives on the device: `position` (int64)
+ * picks the row of the whole cos/sin tables [table_rows, d] (fp32).  A position outside the table gives
+ * NaN in q_out and k_out.
+ */
+int bfly_qk_norm_rope_at(const void* q, const void* k, const void* v, int64_t q_row_stride, int64_t k_row_stride,
+                         int64_t v_row_stride, const void* q_weight, const void* k_weight, const float* cos_table,
+                         const float* sin_table, int64_t table_rows, const int64_t* position, int64_t batch, int hq,
+                         int hkv, int head_dim, float eps, void* q_out, void* k_out, void* v_out,
+                         hipStream_t stream);
+
+/*
  * Device: out [rows, cols] = SiLU(gate) * up, the SwiGLU MLP's product; gate and
  * up rows are in_row_stride elements apart (2 * cols for a fused gate|up
  * projection output).  No counterpart in the reference's own code.

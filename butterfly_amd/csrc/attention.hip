@@ -18,9 +18,9 @@
 //    fp32 softmax with wavefront shuffles between the 4 lane groups.
 //  * page_attn_kernel<D> (page_attn.h): bf16, head_dim 64/128/256, the windows and block sizes that
 //    attn_mfma_kernel does not take; keys in LDS pages under a running softmax.
-//  * attn_f32_tile_kernel<D>: fp32, head_dim 64/128, W <= 64, GQA groups of at
+//  * attn_f32_tile_kernel<D, WMAX>: fp32, head_dim 64/128, W <= 128, GQA groups of at
 //    most 4, BS a multiple of 16; one workgroup per (batch, kv head, 16-query
-//    tile), keys staged in LDS, both products on v_mfma_f32_16x16x4_f32.
+//    tile), keys staged in LDS, both products on bf16 MFMA over three-part splits.
 //  * attn_generic_kernel<T>: fp32 or bf16, any shape; one wave per
 //    (batch, kv head, query); lanes over keys for scores and over d for output.
 #include <stdlib.h>
@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a) {
 }
 
 // --------------------------------------------------------------------------------------------
-// fp32 tile kernel: contiguous query ranges, W <= 64, d in {64, 128}, GQA groups of at most 4
+// fp32 tile kernel: contiguous query ranges, W <= 128, d in {64, 128}, GQA groups of at most 4
 // heads, block_size % 16 == 0, neighbour rows from a table with 1 <= kcap <= 16.  One 256-thread
 // workgroup per (batch, kv head, 16-query tile at positions 16k .. 16k + 15); wave w computes
 // query head w of the group.  The tile's key rows: the window [k0, k0 + 16 nwt) covering
@@ -283,11 +283,17 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a) {
 //     row-major V parts by transposing LDS reads (pieces swizzled by row).  Output tile (mt, half)
 //     row r is d = 32 mt + 8 (r / 4) + 4 half + r % 4, so each lane ends with 8 consecutive d of
 //     its query per mt.
+// WMAX 64 or 128: the window tiles staged, five or nine.  WMAX 128 (130 KB at d = 128: one workgroup per CU)
+// took the windows above 64 over from attn_generic_kernel, and keeps to its errors: eight part products
+// (all but |al bl| < 2^-28 |a b|), the softmax exponent in one fma, infinities and NaN key by key
+// (f32_rows_plainly).  Over 3 draws of 5 shapes against 64 bits: rms 3.7e-8..5.5e-8 where the generic
+// kernel has 4.9e-8..7.1e-8, the largest single error 1.75e-6 against 1.73e-6.  Calls of 4096 tokens, 8/2
+// heads of d 128: W = 128 303 -> 55 us, W = 65 184 -> 55 us; one row over such a cache, W = 128,
+// 84 -> 44 us (the calls' host part included): the rule needs no lower limit on the rows.
 // Positions and ring slots are 32-bit (the host sends only caches and rings below 2^30 rows here).
 constexpr int kF32MaxKcap = 16;
-constexpr int kF32WinTiles = 5;        // (64 - 1 + 15) / 16 + 1
-constexpr int kF32Tiles = kF32WinTiles + 1;
-constexpr int kF32Rows = 16 * kF32Tiles;
+constexpr int f32_win_tiles(int W) { return (W - 1 + 15) / 16 + 1; }   // 5 for 64, 9 for 128
+constexpr int f32_rows(int W) { return 16 * (f32_win_tiles(W) + 1); }
 
 // The three bf16 parts (bit patterns, two per dword, element 0 in the low half) of four floats.
 struct Parts4 {
@@ -319,8 +325,102 @@ __device__ __forceinline__ f32x4 mfma_x6(const bf16x8 (&a)[3], const bf16x8 (&b)
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], c, 0, 0, 0);
 }
 
+// The 16 queries of a tile and one head per wave, key by key in fp32 as attn_generic_kernel does it,
+// for tiles whose rows or scores hold an infinity or NaN: those do not survive the split into parts
+// (inf - inf) and, as 0 * NaN, would reach queries whose window does not hold them.  Every wave of the
+// workgroup calls it (barriers); `ps`: the wave's WMAX + 16 floats of LDS.
 template <int D>
-__global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int tile0, int ntiles, int per_xcd) {
+__device__ void f32_rows_plainly(const AttnArgs& a, int64_t bi, int kvh, int hq_i, bool store, int q0, int lane,
+                                 int nb_lane, int blk, float* ps) {
+  const int64_t row0 = bi * a.hkv + kvh;
+  const float* kb = reinterpret_cast<const float*>(a.k) + row0 * a.kv_rows * D;
+  const float* vb = reinterpret_cast<const float*>(a.v) + row0 * a.kv_rows * D;
+  const float* ksb = reinterpret_cast<const float*>(a.ks) + row0 * a.pool_rows * D;
+  const float* vsb = reinterpret_cast<const float*>(a.vs) + row0 * a.pool_rows * D;
+#pragma unroll 1
+  for (int r = 0; r < 16; ++r) {
+    const int p = q0 + r;
+    if (p < a.q_pos0 || p >= a.q_pos0 + a.tq) continue;      // the same for every wave
+    const int lo = max(max(p - a.W + 1, (int)a.key_lo), 0), hi = min(p, (int)a.kv_len - 1);
+    const int nw = max(hi - lo + 1, 0), nk = nw + kF32MaxKcap;
+    const int cut = max((a.token_cutoff ? p : blk * a.bs) - a.W + 1, 0);
+    const int64_t qoff = ((bi * a.hq + hq_i) * a.tq + (p - a.q_pos0)) * D;
+    const float* q = reinterpret_cast<const float*>(a.q) + qoff;
+    // row of key idx (window, then summary slots); false for an unused slot.  Every lane calls it.
+    auto key = [&](int idx, bool v, const float*& x) {
+      const int n = __shfl(nb_lane, max(idx - nw, 0) & 15);
+      if (idx < nw) {
+        const int pos = lo + idx;
+        x = (v ? vb : kb) + (int64_t)(a.ring ? (int)((uint32_t)pos % (uint32_t)a.ring) : pos - (int)a.key_lo) * D;
+        return true;
+      }
+      x = (v ? vsb : ksb) + (int64_t)max(n, 0) * D;
+      return idx < nk && n >= 0 && (n + 1) * a.bs <= cut;
+    };
+    __syncthreads();                                         // the scores of the row before are read
+    float mx = -INFINITY;
+#pragma unroll 1
+    for (int base = 0; base < nk; base += 64) {
+      const float* x;
+      const int idx = base + lane;
+      const bool ok = key(idx, false, x);
+      float s = 0.f;
+      if (ok) {
+#pragma unroll 1
+        for (int c = 0; c < D; ++c) s = fmaf(q[c], x[c], s);
+        s *= a.scale;
+        mx = fmaxf(mx, s);
+      }
+      if (idx < nk) ps[idx] = s;
+    }
+    mx = wave_max(mx);
+    float l = 0.f;
+#pragma unroll 1
+    for (int base = 0; base < nk; base += 64) {
+      const float* x;
+      const int idx = base + lane;
+      const bool ok = key(idx, false, x);
+      if (idx < nk) {
+        const float e = ok ? expf(ps[idx] - mx) : 0.f;
+        ps[idx] = e;
+        l += e;
+      }
+    }
+    const float inv = 1.f / fmaxf(wave_sum(l), 1e-9f);
+    __syncthreads();
+    float acc[D / 64];
+#pragma unroll
+    for (int c = 0; c < D / 64; ++c) acc[c] = 0.f;
+#pragma unroll 1
+    for (int idx = 0; idx < nk; ++idx) {
+      const float* x;
+      if (!key(idx, true, x)) continue;                      // the same for every lane
+      const float e = ps[idx];
+#pragma unroll
+      for (int c = 0; c < D / 64; ++c) acc[c] = fmaf(e, x[lane + 64 * c], acc[c]);
+    }
+    if (store) {
+#pragma unroll
+      for (int c = 0; c < D / 64; ++c) reinterpret_cast<float*>(a.out)[qoff + lane + 64 * c] = acc[c] * inv;
+    }
+  }
+}
+
+// c + a b with the two products of mid and lo parts as well (kExact): what is dropped is |al bl| < 2^-28 |a b|
+template <bool kExact>
+__device__ __forceinline__ f32x4 mfma_parts(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x4 c) {
+  if constexpr (kExact) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[1], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[2], c, 0, 0, 0);
+  }
+  return mfma_x6(a, b, c);
+}
+
+template <int D, int WMAX>
+__global__ void __launch_bounds__(256, WMAX > 64 && D > 64 ? 1 : 2)
+attn_f32_tile_kernel(AttnArgs a, int tile0, int ntiles, int per_xcd) {
+  constexpr bool kWide = WMAX > 64;
+  constexpr int kF32WinTiles = f32_win_tiles(WMAX), kF32Tiles = kF32WinTiles + 1, kF32Rows = f32_rows(WMAX);
   constexpr int DG = D / 4;                                 // d per lane group
   constexpr int KP = D + 8;                                 // K part row pitch (bf16; 16-byte pad)
   constexpr int KSTEPS = D / 32;
@@ -333,7 +433,17 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
   static_assert(256 % PER_ROW == 0 && 16 % RSTEP == 0, "a thread's pieces are one column, RSTEP rows apart");
   static_assert(kF32Tiles % 2 == 0, "key tiles are scored in pairs");
   __shared__ __attribute__((aligned(16))) __bf16 lds[3 * KPART];   // K parts, then V parts
+  // kWide: an infinity or NaN among the rows read or the scores (see f32_rows_plainly)
+  __shared__ int s_bad;
+  float watch = 0.f;      // NaN as soon as it has seen one
+  auto see = [&](f32x4 x) {
+    if constexpr (kWide) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) watch = fmaf(x[i], 0.f, watch);
+    }
+  };
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  if (kWide && tid == 0) s_bad = 0;
   // workgroups are dispatched to the 8 XCDs round-robin: XCD x = blockIdx % 8 takes the items
   // x per_xcd .. x per_xcd + per_xcd - 1, consecutive tiles of one (batch, kv head), which share
   // most of their window rows in that XCD's L2
@@ -420,12 +530,16 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
   const int cut = max(a.token_cutoff ? p - W + 1 : blk * bs - W + 1, 0);
   const int klo = max(max(p - W + 1, key_lo), 0), khi = min(p, kv_len - 1);
   const float sl2 = a.scale * 1.4426950408889634f;          // scale * log2(e)
+  // what sl2 leaves of it: the product's rounding and log2(e) - float(log2(e))
+  [[maybe_unused]] const float sl2_lo = fmaf(a.scale, 1.4426950408889634f, -sl2) + a.scale * 1.925963e-8f;
 
   // Q's parts in MFMA B-operand form: k-step ks holds d = DG lg + 8 ks + 0..7
   bf16x8 qf[KSTEPS][3];
 #pragma unroll
   for (int ks = 0; ks < KSTEPS; ++ks) {
     const Parts4 x0 = split_parts(qv[2 * ks]), x1 = split_parts(qv[2 * ks + 1]);
+    see(qv[2 * ks]);
+    see(qv[2 * ks + 1]);
     qf[ks][0] = join8(x0.h, x1.h);
     qf[ks][1] = join8(x0.m, x1.m);
     qf[ks][2] = join8(x0.l, x1.l);
@@ -439,6 +553,7 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
 #pragma unroll
     for (int u = t0 * UPT; u < (t0 + 2) * UPT; ++u) {
       const Parts4 x = split_parts(kx[u]);
+      see(kx[u]);
       const int off = (row0 + RSTEP * u) * KP + 4 * c4;
       *reinterpret_cast<uint2*>(lds + off) = x.h;
       *reinterpret_cast<uint2*>(lds + KPART + off) = x.m;
@@ -453,10 +568,12 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
         const bf16x8 kf[3] = {*reinterpret_cast<const bf16x8*>(lds + off),
                               *reinterpret_cast<const bf16x8*>(lds + KPART + off),
                               *reinterpret_cast<const bf16x8*>(lds + 2 * KPART + off)};
-        c[t] = mfma_x6(kf, qf[ks], c[t]);
+        c[t] = mfma_parts<kWide>(kf, qf[ks], c[t]);
       }
     }
   }
+#pragma unroll
+  for (int t = 0; t < kF32Tiles; ++t) see(c[t]);
   float sc[kF32Tiles][4];
   float m = -INFINITY;
 #pragma unroll
@@ -481,7 +598,14 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
   for (int t = 0; t < kF32Tiles; ++t)
 #pragma unroll
     for (int jj = 0; jj < 4; ++jj) {
-      sc[t][jj] = __builtin_amdgcn_exp2f(sc[t][jj] - m);   // exp2(-inf) = 0
+      // (kWide: the exponent c scale log2(e) - m with the factor in two parts and no rounding of the
+      // product, since a rounded one is off by 2^-24 of itself and not of the difference)
+      if constexpr (kWide) {
+        const float e = fmaf(c[t][jj], sl2, fmaf(c[t][jj], sl2_lo, -m));
+        sc[t][jj] = sc[t][jj] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(e);
+      } else {
+        sc[t][jj] = __builtin_amdgcn_exp2f(sc[t][jj] - m);   // exp2(-inf) = 0
+      }
       l += sc[t][jj];
     }
   l += __shfl_xor(l, 16);
@@ -501,13 +625,22 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
 #pragma unroll
   for (int u = 0; u < STAGE; ++u) {
     const Parts4 x = split_parts(vx[u]);
+    see(vx[u]);
     const int row = row0 + RSTEP * u;
     const int off = row * D + (c4 ^ (2 * vrow_swizzle<D>(row))) * 4;
     *reinterpret_cast<uint2*>(lds + off) = x.h;
     *reinterpret_cast<uint2*>(lds + VPART + off) = x.m;
     *reinterpret_cast<uint2*>(lds + 2 * VPART + off) = x.l;
   }
+  if (kWide && watch != watch) s_bad = 1;   // (cleared before K's barriers)
   __syncthreads();   // V parts in LDS
+  if constexpr (kWide) {
+    if (s_bad) {
+      f32_rows_plainly<D>(a, bi, kvh, hq_i, w < gsz, q0, lane, nb_lane, blk,
+                          reinterpret_cast<float*>(lds) + w * (WMAX + kF32MaxKcap));
+      return;
+    }
+  }
 
   const float inv = 1.f / fmaxf(l, 1e-9f);
   float* op = reinterpret_cast<float*>(a.out) + ((bi * a.hq + hq_i) * a.tq + qrow) * D + 8 * lg;
@@ -530,7 +663,7 @@ __global__ void __launch_bounds__(256, 2) attn_f32_tile_kernel(AttnArgs a, int t
         for (int pt = 0; pt < 3; ++pt)
           vf[pt] = __builtin_shufflevector(read_tr(lds + pt * VPART + oa), read_tr(lds + pt * VPART + ob), 0, 1, 2,
                                            3, 4, 5, 6, 7);
-        acc = mfma_x6(vf, pf[pr], acc);
+        acc = mfma_parts<kWide>(vf, pf[pr], acc);
       }
       o[half] = acc;
     }
@@ -1475,10 +1608,10 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
       launch_win_attn<kPageFused>(page_args(a), a.d, stream);
     else
       launch_page_attn<kPageFused>(page_args(a), a.d, stream);
-  } else if (dtype == BFLY_DTYPE_F32 && contiguous && a.nbr != nullptr && a.W <= 64 && a.bs % 16 == 0 &&
+  } else if (dtype == BFLY_DTYPE_F32 && contiguous && a.nbr != nullptr && a.W <= 128 && a.bs % 16 == 0 &&
              a.hq / a.hkv <= 4 &&
              (a.d == 64 || a.d == 128) && a.kcap >= 1 && a.kcap <= kF32MaxKcap &&
-             a.kv_len + 2 * kF32Rows < (1 << 30) && a.ring < (1 << 30) && a.nblocks >= 1 &&
+             a.kv_len + 2 * f32_rows(128) < (1 << 30) && a.ring < (1 << 30) && a.nblocks >= 1 &&
              a.nblocks * (int64_t)a.bs < (1 << 30) &&
              a.q_pos0 >= 0 && a.q_pos0 + a.tq < (1 << 30) && a.pool_rows > 0) {
     const int64_t tile0 = floordiv(a.q_pos0, 16);
@@ -1487,10 +1620,9 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
     const int64_t per_xcd = (items + 7) / 8;
     BFLY_CHECK_ARG(8 * per_xcd <= INT32_MAX, "%s: grid too large", what);
     const dim3 grid((unsigned)(8 * per_xcd));
-    if (a.d == 64)
-      hipLaunchKernelGGL(attn_f32_tile_kernel<64>, grid, dim3(256), 0, stream, a, (int)tile0, (int)ntiles, (int)per_xcd);
-    else
-      hipLaunchKernelGGL(attn_f32_tile_kernel<128>, grid, dim3(256), 0, stream, a, (int)tile0, (int)ntiles, (int)per_xcd);
+    auto kernel = a.W <= 64 ? (a.d == 64 ? attn_f32_tile_kernel<64, 64> : attn_f32_tile_kernel<128, 64>)
+                            : (a.d == 64 ? attn_f32_tile_kernel<64, 128> : attn_f32_tile_kernel<128, 128>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, (int)tile0, (int)ntiles, (int)per_xcd);
   } else {
     BFLY_CHECK_ARG(a.d <= kGenericMaxD, "%s: head_dim=%d > %d", what, a.d, kGenericMaxD);
     BFLY_CHECK_ARG(a.W + a.kcap <= kGenericMaxKeys, "%s: window + kcap > %d", what, kGenericMaxKeys);

@@ -1,0 +1,90 @@
+"""GPU: fp32 windows of 65 to 128 tokens on the tile kernel, against a 64-bit softmax.
+
+Bound: a score q.k * scale sums D products of which the split drops at most 2^-28 |q_i k_i| and the
+fp32 accumulation rounds by at most D 2^-24: with sum |q_i k_i| * scale <= 12 for these inputs less than
+12 (2^-28 + 2^-17) = 9.2e-5 (worst signs), which is the weights' relative error; values reach 5 and the
+weights sum to 1, so the mean over keys is off by less than 4.6e-4; rounding errors of random sign leave
+less than an eighth of it.
+"""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+import butterfly_amd as bf
+from oracle import topology as tp
+
+pytestmark = pytest.mark.gpu
+
+ABS = 5.5e-5
+
+
+def _rand(seed, *shape):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed))
+
+
+def _want(q, k, v, ks, vs, row, p, w, bs, cut, nsum, scale):
+    blk, lo = p // bs, max(0, p - w + 1)
+    sel = [n for n in row if 0 <= n < blk and n < nsum and (n + 1) * bs <= cut]
+    keys, vals = torch.cat([k[lo:p + 1], ks[sel]]).double(), torch.cat([v[lo:p + 1], vs[sel]]).double()
+    return torch.softmax(keys @ q.double() * scale, 0) @ vals
+
+
+# b, hq, hkv, t, d, bs, W: window edges, lengths off the 16-row tile, GQA groups of 1 to 4
+CASES = [(1, 1, 1, 1, 64, 64, 65), (1, 4, 1, 333, 128, 64, 65), (2, 3, 1, 500, 64, 128, 127),
+         (1, 4, 2, 777, 128, 128, 128), (1, 2, 1, 450, 128, 48, 97), (1, 3, 1, 290, 64, 16, 128)]
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("case", CASES)
+def test_prefill(case, special):
+    b, hq, hkv, t, d, bs, w = case
+    g = hq // hkv
+    q, k, v = _rand(1, b, hq, t, d), _rand(2, b, hkv, t, d), _rand(3, b, hkv, t, d)
+    if special and t > 250:
+        v[0, 0, 130, 3], v[0, 0, 201, d - 1], v[0, 0, 207] = math.inf, -math.inf, math.nan
+        k[0, 0, 240, 0] = math.inf
+    kw = dict(seq_len=t, block_size=bs, num_key_value_heads=hkv, num_key_value_groups=g, layer_idx=2,
+              local_window_blocks=1, sink_count=1, partner_count=1, partner_rule="xor")
+    got = bf.compressed_butterfly_attention(q.cuda(), k.cuda(), v.cuda(), layout=bf.build_block_butterfly_layout(**kw),
+                                            local_window_tokens=w)[0].cpu().double()
+    ks, vs = (s.cpu() for s in bf.block_mean_summaries(k.cuda(), seq_len=t, block_size=bs, num_blocks=-(-t // bs),
+                                                       x2=v.cuda()))
+    rows = tp.build_layout(**kw).block_neighbors[0]
+    for bi in range(b):
+        for h in range(hq):
+            kv = h // g
+            want = torch.stack([_want(q[bi, h, p], k[bi, kv], v[bi, kv], ks[bi, kv], vs[bi, kv],
+                                      rows[p // bs].tolist(), p, w, bs, max(0, p // bs * bs - w + 1), 1 << 30, d ** -0.5)
+                                for p in range(t)])
+            assert torch.equal(torch.isnan(got[bi, h]), torch.isnan(want))
+            assert torch.equal(torch.isinf(got[bi, h]), torch.isinf(want))
+            fin = torch.isfinite(want)
+            assert (got[bi, h] - want)[fin].abs().max() <= ABS
+
+
+@pytest.mark.parametrize("d,w,step,hq,hkv", [(64, 100, 37, 2, 2), (128, 128, 70, 4, 1), (128, 65, 1, 3, 1)])
+def test_ring_chunks(d, w, step, hq, hkv):
+    bs, t, g = 64, 700, hq // hkv
+    q, k, v = _rand(1, 1, hq, t, d), _rand(2, 1, hkv, t, d), _rand(3, 1, hkv, t, d)
+    cache = bf.CompressedKVCache(block_size=bs, local_window_tokens=w, max_kv_size=t, max_chunk_size=128)
+    start = 0
+    while start < t:
+        n = min(step if start or step > 1 else 128, t - start) if start < 200 or step > 1 else min(step, t - start)
+        n = min(n, 3) if step == 1 and start > 400 else n
+        kw = dict(seq_len=start + n, block_size=bs, num_key_value_heads=hkv, num_key_value_groups=g, layer_idx=1,
+                  local_window_blocks=1, sink_count=1, partner_count=1, partner_rule="causal_shift")
+        s = slice(start, start + n)
+        got = cache.update_and_attend(q[:, :, s].cuda(), k[:, :, s].cuda(), v[:, :, s].cuda(),
+                                      layout=bf.build_block_butterfly_layout(**kw), local_window_tokens=w).cpu().double()
+        rows, pk, pv = tp.build_layout(**kw).block_neighbors[0], cache._pool_k.cpu(), cache._pool_v.cpu()
+        for i, p in enumerate(range(start, start + n)):
+            if n > 5 and i % 9 and i != n - 1:
+                continue
+            for h in range(hq):
+                want = _want(q[0, h, p], k[0, h // g], v[0, h // g], pk[0, h // g], pv[0, h // g], rows[p // bs].tolist(),
+                             p, w, bs, max(0, p - w + 1), cache.summary_count, d ** -0.5)
+                assert (got[0, h, i] - want).abs().max() <= ABS, p
+        start += n

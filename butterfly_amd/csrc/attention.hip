@@ -1978,10 +1978,13 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // Wide batches leave the tokens below their tail out of the ring; the call's last launch copies
   // those that its last ring_capacity positions hold (copy_rest), so that the whole ring is what one
   // chunk per batch leaves.  A W <= 64 call whose chunks share batches under the length rule keeps
-  // that rule alone (its batches copy only their tails).
-  bool wide = true;
+  // that rule alone (its batches copy only their tails), and so does one with a chunk off the page grid,
+  // which no wide batch holds: 9000 tokens of d 256 in chunks of 700, 251 us, 262 with the copies
+  // alone.  In chunks of 512, 20000 tokens of d 256, 16/4 heads, window 64: 630 us by length, 327 wide;
+  // of 1024, 30000 tokens of d 64, 8/4 heads: 400 and 203.
+  bool wide = paged || s.offset % kPage == 0;
   for (int64_t c = 0; !paged && c + 1 < n_chunks; ++c)
-    if (chunk_len[c] + chunk_len[c + 1] <= budget) wide = false;
+    if (chunk_len[c] + chunk_len[c + 1] <= budget || chunk_len[c] % kPage != 0) wide = false;
   const int64_t call_offset = s.offset;
   auto plan_batch = [&](const StreamCounters& s0, int64_t from, Batch& bt) -> int {
     bt = Batch{};

@@ -237,26 +237,19 @@ def _positions(query_positions, tq: int, device):
     return 0, qp.to(device=device, dtype=torch.int32)
 
 
-def decode_row_entry(tensors, *, rows: int, ring_capacity: int, kv_len: int, pool_rows: int, num_blocks: int,
-                     block_size: int, window: int, row_slots: int, scale: float) -> Optional[str]:
-    """The fused entry that takes one new row per sequence, or ``None`` for the general path.
+def decode_wide_fits(tensors, *, rows: int, ring_capacity: int, kv_len: int, pool_rows: int, num_blocks: int,
+                     block_size: int, window: int, scale: float) -> bool:
+    """Whether one new row per sequence over a window above 64 tokens goes to ``bfly_decode_wide``: bf16 windows
+    of up to 128, the last that its 144 staged keys hold, within its limits (32-bit offsets, 16-byte pieces, a
+    table that covers the position), which the general path does not have.
 
-    ``tensors``: the query first, then the ring (or tail) and pool.  Head_dim 64 or 128 (256 for bf16) and a
-    routed row of at most 16 slots: ``bfly_decode`` for windows of up to 64 tokens, ``bfly_decode_wide`` for
-    bf16 windows of 65 to 128, the last that its 144 staged keys hold.  The wide kernel's limits (32-bit offsets,
-    16-byte pieces, a table that covers the position) are checked here: the general path has none of them.
+    ``tensors``: the query first, then the ring (or tail) and pool.
     """
     q = tensors[0]
-    d, bf16 = int(q.shape[3]), q.dtype == torch.bfloat16
-    if row_slots > 16 or not (d in (64, 128) or (d == 256 and bf16)):
-        return None
-    if window <= 64:
-        return "bfly_decode"
-    lim = 1 << 30
-    wide = (bf16 and window <= 128 and scale > 0.0 and rows * d < lim and pool_rows * d < lim and ring_capacity < lim
-            and kv_len < lim and num_blocks < lim and num_blocks * block_size >= kv_len
+    d, lim = int(q.shape[3]), 1 << 30
+    return (q.dtype == torch.bfloat16 and window <= 128 and scale > 0.0 and rows * d < lim and pool_rows * d < lim
+            and ring_capacity < lim and kv_len < lim and num_blocks < lim and num_blocks * block_size >= kv_len
             and all(t.data_ptr() % 16 == 0 for t in tensors))
-    return "bfly_decode_wide" if wide else None
 
 
 def _attend(q, tail_k, tail_v, pool_k, pool_v, *, layout, q_pos0, qpos_dev, ring_capacity, tail_start,
@@ -265,17 +258,17 @@ def _attend(q, tail_k, tail_v, pool_k, pool_v, *, layout, q_pos0, qpos_dev, ring
     hk = tail_k.shape[1]
     out = torch.empty_like(q)
     nb = layout.neighbors
-    entry = None
+    w = int(local_window_tokens)
     if (tq == 1 and qpos_dev is None and int(q_pos0) == int(kv_len) - 1 and int(tail_start) < int(kv_len)
-            and pool_k.shape[2] > 0):
-        entry = decode_row_entry((q, tail_k, tail_v, pool_k, pool_v), rows=tail_k.shape[2],
-                                 ring_capacity=int(ring_capacity), kv_len=int(kv_len), pool_rows=pool_k.shape[2],
-                                 num_blocks=nb.shape[0], block_size=layout.block_size,
-                                 window=int(local_window_tokens), row_slots=nb.shape[1], scale=_scale(scale, d))
-    if entry is not None:
+            and nb.shape[1] <= 16 and pool_k.shape[2] > 0
+            and (d in (64, 128) or (d == 256 and q.dtype == torch.bfloat16))
+            and (w <= 64 or decode_wide_fits((q, tail_k, tail_v, pool_k, pool_v), rows=tail_k.shape[2],
+                                             ring_capacity=int(ring_capacity), kv_len=int(kv_len),
+                                             pool_rows=pool_k.shape[2], num_blocks=nb.shape[0],
+                                             block_size=layout.block_size, window=w, scale=_scale(scale, d)))):
         # a single row at the newest position: the decode kernel
         with _on(q.device):
-            _native.call(entry, q.data_ptr(), _dtype_code(q), b, hq, hk, d, None, None,
+            _native.call("bfly_decode" if w <= 64 else "bfly_decode_wide", q.data_ptr(), _dtype_code(q), b, hq, hk, d, None, None,
                          tail_k.data_ptr(), tail_v.data_ptr(), int(ring_capacity), int(tail_start), int(kv_len),
                          pool_k.data_ptr(), pool_v.data_ptr(), pool_k.shape[2], int(summary_count),
                          layout.table.topology, nb.shape[0], layout.block_size, int(local_window_tokens),

@@ -414,7 +414,7 @@ class CompressedKVCache:
         as one fused launch (append + attention; plus the block compressor on the
         steps that complete a block); longer steps append, then attend.
         """
-        from .attention import _attend, _require_cuda, _scale, decode_row_entry
+        from .attention import _attend, _require_cuda, _scale, decode_wide_fits
 
         _require_cuda(q)
         self.sync()
@@ -422,19 +422,20 @@ class CompressedKVCache:
         d = int(q.shape[3])
         w = int(local_window_tokens)
         nb = layout.neighbors
-        entry = None
-        if step == 1 and int(q.shape[2]) == 1 and q.dtype == keys.dtype:
-            made = self._ring_k is not None
-            # above 64, the general path's fewer conditions: a first step (no buffers yet), other shapes than the
+        fused = (step == 1 and int(q.shape[2]) == 1 and q.dtype == keys.dtype
+                 and nb.shape[1] <= 16
+                 and (d in (64, 128) or (d == 256 and q.dtype == torch.bfloat16)))
+        if fused and w > 64:
+            # the general path has fewer conditions: a first step (no buffers yet), other shapes than the
             # keys' and a cache that pools the newest block go there
-            if w <= 64 or (made and self.local_window_tokens > 0 and q.shape[0] == keys.shape[0]
-                           and d == keys.shape[3] == values.shape[3]):
-                bufs = (self._ring_k, self._ring_v, self._pool_k, self._pool_v) if made else ()
-                entry = decode_row_entry((q, *bufs), rows=self.tail_capacity, ring_capacity=self.tail_capacity,
-                                         kv_len=self.offset + 1, pool_rows=self.summary_capacity,
-                                         num_blocks=nb.shape[0], block_size=layout.block_size, window=w,
-                                         row_slots=nb.shape[1], scale=_scale(scale, d))
-        if entry is None:
+            fused = (self._ring_k is not None and self.local_window_tokens > 0 and q.shape[0] == keys.shape[0]
+                     and d == keys.shape[3] == values.shape[3]
+                     and decode_wide_fits((q, self._ring_k, self._ring_v, self._pool_k, self._pool_v),
+                                          rows=self.tail_capacity, ring_capacity=self.tail_capacity,
+                                          kv_len=self.offset + 1, pool_rows=self.summary_capacity,
+                                          num_blocks=nb.shape[0], block_size=layout.block_size, window=w,
+                                          scale=_scale(scale, d)))
+        if not fused:
             self.update(keys, values)
             return _attend(_c(q), self._ring_k, self._ring_v, self._pool_k, self._pool_v, layout=layout,
                            q_pos0=self.offset - int(q.shape[2]), qpos_dev=None, ring_capacity=self.tail_capacity,
@@ -452,7 +453,7 @@ class CompressedKVCache:
         b, hq = int(q.shape[0]), int(q.shape[1])
         out = torch.empty_like(q)
         with _on(q.device):
-            _native.call(entry, q.data_ptr(), _dtype_code(q), b, hq, int(keys.shape[1]), d,
+            _native.call("bfly_decode" if w <= 64 else "bfly_decode_wide", q.data_ptr(), _dtype_code(q), b, hq, int(keys.shape[1]), d,
                          keys.data_ptr(), values.data_ptr(), self._ring_k.data_ptr(), self._ring_v.data_ptr(),
                          self.tail_capacity, self.offset - self.tail_size, self.offset, self._pool_k.data_ptr(),
                          self._pool_v.data_ptr(), self.summary_capacity, self.summary_count, layout.table.topology,

@@ -149,15 +149,20 @@ class QuantLinear(nn.Module):
         return self.group % Q4_PIECE_CODES == 0 and self.in_features <= Q4_MAX_IN
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if _one_row(x) and self.gemv_from_codes:
-            return q4_gemv(x, self)
-        if q4_rows_fits(x, self):
-            return q4_rows(x, self)
+        if x.numel() <= Q4_MAX_ROWS * x.shape[-1]:
+            if _one_row(x) and self.gemv_from_codes:
+                return q4_gemv(x, self)
+            if q4_rows_fits(x, self):
+                return q4_rows(x, self)
         return _linear(x, self.weight)
 
 
 # shape limits of bfly_q4_gemv / bfly_q4_gemv_silu (include/butterfly_amd_decoder.h)
 Q4_PIECE_CODES, Q4_MAX_IN = 32, 8192
+# rows that a product from the codes takes at most (q4_rows_fits); one test of it turns a prefill's layers
+# away from every few-row path (335 tokens through four layers, host-bound: 952 us before there was a few-row
+# path, 1042 with its whole rule tested by every layer, level with 952 so)
+Q4_MAX_ROWS = 32
 # decode steps of a swapped layer run its output projection in the decode-step launch where
 # the shapes allow (ButterflyAttention.takes_o_proj); False keeps it a launch of its own
 FUSE_O_PROJ = True
@@ -211,12 +216,11 @@ def q4_rows_fits(x: torch.Tensor, layer: QuantLinear) -> bool:
     rows the GEMM is faster, and from 17 rows on for more than 4096 inputs (6144 x 2048, 17 rows:
     12.6 against 11.7)."""
     n = layer.in_features
+    if not 2 * n <= x.numel() <= (16 if n > 4096 else Q4_MAX_ROWS) * n:
+        return False
     if type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.bfloat16 or x.shape[-1] != n \
             or n % 256 or layer.group != 64 or layer.packed.device != x.device \
             or (layer.packed.data_ptr() | layer.scale_bias.data_ptr()) % 16:
-        return False
-    rows = x.numel() // n
-    if not 2 <= rows <= (16 if n > 4096 else 32):
         return False
     return not (torch.is_grad_enabled() and x.requires_grad) and torch.autograd.forward_ad._current_level < 0 \
         and not torch._C._functorch.is_functorch_wrapped_tensor(x)
@@ -635,10 +639,11 @@ class MLP(nn.Module):
         self.gate_up = QuantLinear.fuse_rows(self.gate_proj, self.up_proj)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if _one_row(x) and self.gate_up.gemv_from_codes:
-            return self.down_proj(q4_gemv_silu(x, self.gate_up))
-        if q4_rows_fits(x, self.gate_up):
-            return self.down_proj(q4_rows_silu(x, self.gate_up))
+        if x.numel() <= Q4_MAX_ROWS * x.shape[-1]:
+            if _one_row(x) and self.gate_up.gemv_from_codes:
+                return self.down_proj(q4_gemv_silu(x, self.gate_up))
+            if q4_rows_fits(x, self.gate_up):
+                return self.down_proj(q4_rows_silu(x, self.gate_up))
         if _hip(x):
             gu = self.gate_up(x)                           # [..., 2f]: gate columns, then up columns
             f = gu.shape[-1] // 2

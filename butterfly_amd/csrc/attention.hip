@@ -1517,8 +1517,8 @@ static int chunk_blocks_max(int bs) { return bs % kPageRows == 0 ? 1 : kPageRows
 // Whether the paged kernel takes a bf16 launch over contiguous positions: its summary page holds 64
 // slots (the routed rows of every block that 64 positions touch), a ring page may wrap once,
 // positions are 32-bit.  It replaces the generic kernel wherever it can run: the one-shot call over
-// 2 x 10007 tokens, 16 query heads over 4 of d 128, W 128 took 1711 us there and takes 109 us here,
-// one decode row over a 128-token window 81 us (host work included) and 21 us.
+// 2 x 10007 tokens, 16 query heads over 4 of d 128, W 128 took 1711 us there and 109 us here (78 on
+// win_attn_kernel, which has the windows of 65..128 where the grid fills the chip).
 static bool page_path(const AttnArgs& a, int blocks) {
   return (a.d == 64 || a.d == 128 || a.d == 256) && a.W + (int64_t)a.kcap <= kGenericMaxKeys &&
          blocks * (int64_t)a.kcap <= kPageRows && (a.ring == 0 || a.ring >= kPageRows) && a.q_pos0 >= 0 &&
@@ -1962,7 +1962,8 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // tokens than the ring, as long as no slot that is written is one that the update pools from or
   // the attention's halo lies in (ring_disjoint).  With the default ring (1408 rows for 512-token chunks
   // and 128-token windows) that is ten chunks a launch instead of one: 20011 tokens of d 256, 16
-  // query heads over 4, 1812 us a stream with a launch per chunk, 407 so.
+  // query heads over 4, window 128: 1812 us a stream with a launch per chunk, 407 so, both on
+  // page_attn_kernel (288 on win_attn_kernel).
   struct Batch {
     int64_t first = 0, count = 0, total = 0;
     AttnArgs args[kMaxUpdateParts];

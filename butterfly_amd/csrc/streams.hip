@@ -10,7 +10,7 @@
 //
 // bf16 with head_dim 64, 128 or 256 runs on the paged MFMA kernel (page_attn.h): window stream,
 // dense summaries and merge over 8192 tokens, 8 query heads over 2 of d 128, took 680 us on
-// stream_kernel and take 55 us there.
+// stream_kernel and take 47 to 50 us there.
 //
 // stream_kernel (fp32, other head dims): one wave per (batch, query head, query).  Keys are visited in
 // groups of 64 (one per lane) with a running max and rescaled accumulators, so
@@ -191,7 +191,7 @@ __device__ __forceinline__ void load8_f32(const __bf16* p, float (&x)[8]) {
 
 // merge_kernel with eight elements of a row per thread (d a multiple of 8, aligned pointers): the same
 // arithmetic per element.  HBM-bound: both outputs read, fp32 written once.  8192 x 8 rows of 128 in
-// bf16 (67 MB): 26.4 us with an element a thread (64-bit division, two exponentials each), 22 here with its launch gap.
+// bf16 (67 MB): 26.4 us with an element a thread (64-bit division, two exponentials each), 15.7 here (kernel trace).
 template <typename TA, typename TB>
 __global__ void __launch_bounds__(256) merge8_kernel(const TA* __restrict__ oa, const float* __restrict__ la,
                                                      const float* __restrict__ ma, const TB* __restrict__ ob,

@@ -17,6 +17,11 @@
 //
 // An infinity or NaN in V: its rows are flagged when V is staged; a unit with any takes fragments with
 // such elements zeroed and adds them afterwards to the rows that attend to them.
+//
+// What bounds it: the chain request, scores, softmax, V, store within a workgroup (two of them per CU at
+// d = 128), with the VALU about 40% busy.  2 x 10007 tokens, 16/4 heads of d 128, W 128, with the compressor's
+// 8 us: 109 us a call on page_attn_kernel, 78 here (40 by bytes); 20011 tokens of d 256 streamed in
+// chunks of 512: 407 and 288.
 #pragma once
 
 #include "page_attn.h"

@@ -951,9 +951,9 @@ __device__ __forceinline__ void dec_pool32(const DecodeArgs& a, const DecState32
 // bit.  Every attending workgroup of a sequence appends the new token and pools a due
 // block (the same values), so none reads what another writes in the launch.
 // kWin: window rows staged, 64 or (host-counter steps) 128.  The wide form stages 144 keys, nine
-// score tiles and five PV k-steps, and keeps P to fp32's worth in two bf16 parts, hi + lo, as the
-// attention launch that it replaces does.  One sequence, 16/4 heads of 128, window 128, a step with
-// its append: 19.6 us a call; as an update launch and a paged attention launch 22.7 (with a generic
+// score tiles and five PV k-steps, and keeps P whole, all 24 bits of the fp32 value, in three bf16 parts.  One
+// sequence, 16/4 heads of 128, window 128, a step with its append: 19.0 us a call (19.0 with P in two parts, whose
+// 16 or 17 bits moved outputs by a bf16 step; as an update launch and a paged attention launch 22.7, with a generic
 // attention launch 81.6).  It is a chain of latencies: loads, nine score tiles, one softmax, PV.
 template <int D, bool kStep, bool kQkn = false, int kOS = 0, int kWin = kDecMaxWin>
 __global__ void __launch_bounds__(kOS > 0 ? 512 : 256, kQkn || kWin > 64 ? 1 : (D <= 128 ? 3 : 1))
@@ -1284,9 +1284,9 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
     mx = col_max4(mx);
     const float nm = -mx * sl2;                      // nw >= 1: every column has a finite max
     float lsum = 0.f;
-    bf16x8 pf[NPR], pl[kWide ? NPR : 1];
+    bf16x8 pf[NPR], pm[kWide ? NPR : 1], pl[kWide ? NPR : 1];   // kWide: P = pf + pm + pl, exactly
     pf[NPR - 1] = bf16x8{};
-    if constexpr (kWide) pl[NPR - 1] = bf16x8{};
+    if constexpr (kWide) pm[NPR - 1] = pl[NPR - 1] = bf16x8{};
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -1295,7 +1295,12 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
         lsum += e;
         const __bf16 eh = (__bf16)e;
         pf[t / 2][(t % 2) * 4 + i] = eh;
-        if constexpr (kWide) pl[t / 2][(t % 2) * 4 + i] = (__bf16)(e - (float)eh);
+        if constexpr (kWide) {
+          const float r = e - (float)eh;
+          const __bf16 em = (__bf16)r;
+          pm[t / 2][(t % 2) * 4 + i] = em;
+          pl[t / 2][(t % 2) * 4 + i] = (__bf16)(r - (float)em);
+        }
       }
     lsum = col_sum4(lsum);
     const float inv = kWide ? 1.f / fmaxf(lsum, 1e-30f) : __builtin_amdgcn_rcpf(fmaxf(lsum, 1e-30f));
@@ -1323,11 +1328,14 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
           const bf16x4 vb = 2 * pr + 1 < NT ? vfrag(2 * pr + 1) : bf16x4{};
           const bf16x8 vf = __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7);
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[pr], acc, 0, 0, 0);
-          if constexpr (kWide) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[pr], acc, 0, 0, 0);
+          if constexpr (kWide) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pm[pr], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[pr], acc, 0, 0, 0);
+          }
         }
         if constexpr (kWide) {
-          // An infinite V times lo (zero or negative) would turn its infinity into a NaN: such a
-          // tile is summed again with lo against the finite values alone (hi carries the rest).
+          // An infinite V times a lower part (zero or negative) would turn its infinity into a NaN: such a
+          // tile is summed again with the lower parts against the finite values alone (pf carries the rest).
           const float mag = fmaxf(fmaxf(fabsf(acc[0]), fabsf(acc[1])), fmaxf(fabsf(acc[2]), fabsf(acc[3])));
           const bool bad = acc[0] != acc[0] || acc[1] != acc[1] || acc[2] != acc[2] || acc[3] != acc[3];
           if (__any(bad || mag == INFINITY)) {
@@ -1341,6 +1349,7 @@ decode_mfma_kernel(int64_t* state, const void* q, DecodeArgs a, StepArgs sa_in) 
 #pragma unroll
               for (int i = 0; i < 8; ++i)
                 if (!(fabsf((float)vf[i]) < INFINITY)) vf[i] = (__bf16)0.f;
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pm[pr], acc, 0, 0, 0);
               acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[pr], acc, 0, 0, 0);
             }
           }

@@ -98,3 +98,29 @@ def test_general_path_calls_stay_accepted():
         out = cache.update_and_attend(q[:, :, 300:].cuda(), k[:, :, 300:].cuda(), k[:, :, 300:].cuda(), layout=lay,
                                       local_window_tokens=w, scale=scale)
         assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_weights_keep_fp32_precision(d):
+    """Values that cancel under the weights leave the weights' own error: four window rows of each column are
+    chosen so that the weighted sum is next to zero.  Scores near zero keep an fp32 weight within about 2^-24 of
+    itself, and the sums of random sign come to 2^-23 of size = sqrt(sum (p v)^2); weights of 16 bits miss by
+    2^-19.5 of size (rms)."""
+    h, w, bs, prompt = 4, 128, 128, 400
+    q, k, v = _rand(1, 1, h, 1, d) * 0.05, _rand(2, 1, h, prompt + 1, d), _rand(3, 1, h, prompt + 1, d).double()
+    keys = k[0].double()[:, prompt - w + 1:]
+    kw = dict(seq_len=prompt + 1, block_size=bs, num_key_value_heads=h, num_key_value_groups=1, layer_idx=0,
+              local_window_blocks=0, sink_count=0, partner_count=0, partner_rule="xor")     # no summaries
+    p = torch.softmax((keys @ q[0].double().transpose(1, 2))[..., 0] * d ** -0.5, -1)[..., None]    # [h, w, 1]
+    vals = v[0, :, prompt - w + 1:]                                                                # a view
+    for row in (20, 50, 90, 120):
+        vals[:, row] = 0
+        vals[:, row] = (-(p * vals).sum(1) / p[:, row]).bfloat16().double()
+    cache = bf.CompressedKVCache(block_size=bs, local_window_tokens=w, max_kv_size=512)
+    kd, vd = k.cuda(), v.bfloat16().cuda()
+    cache.update(kd[:, :, :prompt], vd[:, :, :prompt])
+    got = cache.update_and_attend(q.cuda(), kd[:, :, prompt:], vd[:, :, prompt:],
+                                  layout=bf.build_block_butterfly_layout(**kw), local_window_tokens=w)
+    want, size = (p * vals).sum(1), (p * vals).pow(2).sum(1).sqrt()
+    off = (got[0, :, 0].cpu().double() - want).abs() - 2.0 ** -8 * want.abs()
+    assert (off / size).max() <= 2.0 ** -20

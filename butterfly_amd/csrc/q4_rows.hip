@@ -67,6 +67,44 @@ __device__ __forceinline__ __bf16 q4_rows_silu(float g, float u) {
   return (__bf16)(sg * (float)(__bf16)u);
 }
 
+// NaN once `z` is one or `v` holds an infinity or NaN, else zero.
+__device__ __forceinline__ float q4_watch(float z, f32x4 v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) z = fmaf(v[i], 0.f, z);
+  return z;
+}
+
+// A tile's products over runs q0, q0 + step, .. with the weights expanded to bf16 (code * scale + bias), as the
+// GEMM over `weight` takes them, for those that the factorised form left infinite or NaN: an infinite x gives
+// inf - inf there (scale * inf + (bias - 16 scale) * inf), and a finite one above about 1e37 overflows the sum with
+// 16 + code.  Looking for them costs a product at most 1%.  x: this lane's activation row, w: its weight row, both from the row's start; every lane calls it.
+__device__ __forceinline__ f32x4 q4_expanded(const __bf16* x, const uint8_t* w, const uint32_t* sb, int lg, int q0,
+                                             int step, int quads) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int q = q0; q < quads; q += step)
+#pragma unroll 1
+    for (int g = 4 * q; g < 4 * q + 4; ++g) {
+      const float scale = __uint_as_float(sb[g] << 16), bias = __uint_as_float(sb[g] & 0xffff0000u);
+      const int at = 64 * g + q4_first(lg);      // 16 inputs: this lane's two k-steps
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const uint32_t codes = *reinterpret_cast<const uint32_t*>(w + (at + 8 * c) / 2);
+        bf16x8 wf;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wf[e] = (__bf16)fmaf((float)((codes >> (4 * e)) & 15u), scale, bias);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(x + at + 8 * c), wf, acc, 0, 0, 0);
+      }
+    }
+  return acc;
+}
+// `plain` where `v` is an infinity or NaN.
+__device__ __forceinline__ f32x4 q4_mend(f32x4 v, f32x4 plain) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = fabsf(v[i]) < INFINITY ? v[i] : plain[i];
+  return v;
+}
+
 struct Q4RowsArgs {
   const __bf16* x;         // [rows, in_f]
   const uint8_t* w;        // [.., in_f / 2]
@@ -76,9 +114,10 @@ struct Q4RowsArgs {
   int64_t n_out, up_off;
 };
 
-// kSilu: tiles 0 .. R/2 - 1 are gate rows, the others the up rows up_off further.
+// kSilu: tiles 0 .. R/2 - 1 are gate rows, the others the up rows up_off further.  (MT = 1: at most 128
+// registers, for two 512-thread workgroups a CU; with one more, gate|up at 8 rows takes 10.1 us instead of 8.5.)
 template <int MT, int R, int S, bool kSilu>
-__global__ void __launch_bounds__(64 * S) q4_rows_kernel(Q4RowsArgs a) {
+__global__ void __launch_bounds__(64 * S, MT == 1 ? 4 : 2) q4_rows_kernel(Q4RowsArgs a) {
   constexpr int OT = kSilu ? R / 2 : R;
   __shared__ __attribute__((aligned(16))) float part[S][R][MT][64][4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -166,6 +205,18 @@ __global__ void __launch_bounds__(64 * S) q4_rows_kernel(Q4RowsArgs a) {
         }
       }
     }
+  }
+  float watch = 0.f;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) watch = q4_watch(watch, acc[r][m]);
+  if (__any(watch != watch)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[r][m] = q4_mend(acc[r][m], q4_expanded(xp[m] - q4_first(lg), wp[r] - 16 * lg, sp[r], lg, wave, S, quads));
   }
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -265,6 +316,12 @@ __global__ void __launch_bounds__(kQ4WideThreads) q4_rows_wide_kernel(Q4RowsArgs
         for (int i = 0; i < 4; ++i) acc[i] = fmaf(scale, t[i], fmaf(b16, xs[i], acc[i]));
       }
     }
+    const float watch = q4_watch(0.f, acc);
+    if (__any(watch != watch)) {
+      const int64_t row = n < a.n_out ? n : a.n_out - 1;
+      acc = q4_mend(acc, q4_expanded(a.x + (int64_t)min(lq, a.rows - 1) * a.in_f, a.w + row * (a.in_f / 2),
+                                     a.sb + row * groups, lg, 0, 1, quads));
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (4 * lg + i < a.rows && n < a.n_out) a.y[(int64_t)(4 * lg + i) * a.n_out + n] = (__bf16)acc[i];
@@ -302,7 +359,10 @@ static int q4_rows_launch(const void* x, int64_t rows, const void* packed, const
     if constexpr (kSilu) {
       return go(q4_rows_kernel<1, 2, 8, true>, 2, 8);
     } else {
-      if (n_out >= 16384 && in_f <= 4096) {      // enough tiles for every wave of the wide form
+      // from 16384 outputs on (2 / 8 / 16 rows, us, weights beyond the caches; this form, then q4_rows_kernel):
+      // 2048 x 16384 10.7 / 11.2 / 11.8, 10.0 / 11.5 / 13.6; 2048 x 32768 12.6 / 13.1 / 13.8, 17.9 / 20.5 / 23.6;
+      // 512 x 16384 4.5 / 4.7 / 4.9, 5.1 / 5.3 / 5.7; 4096 x 16384 17.3 / 17.8 / 19.2, 14.8 / 17.8 / 22.8
+      if (n_out >= 16384 && in_f <= 4096) {
         const int64_t tiles = (n_out + 15) / 16;
         BFLY_CHECK_ARG(tiles <= INT32_MAX / 2, "%s: out_features too large", what);
         hipLaunchKernelGGL(in_f <= 2048 ? q4_rows_wide_kernel<2048> : q4_rows_wide_kernel<4096>, dim3(kQ4WideGrid),

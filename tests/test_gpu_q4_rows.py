@@ -93,3 +93,35 @@ def test_mlp_rows_match_one_by_one():
     one = torch.cat([mlp(r.unsqueeze(0)) for r in x])
     # the rows' inner activations may differ by a bf16 step where the sums' order rounds differently
     assert ((got - one).float().norm() / one.float().norm()).item() <= 2 ** -8
+
+
+@pytest.mark.parametrize("rows,out_f,in_f", [(2, 40, 256), (16, 100, 2304), (17, 33, 1024), (32, 16400, 512),
+                                             (5, 16400, 2048), (16, 16400, 4096)])
+def test_infinities_and_large_values(rows, out_f, in_f):
+    """An infinity or NaN in a row gives what the product over ``weight`` gives, and a row of values near the type's
+    largest stays finite where that product is; the other rows do not change."""
+    layer = _layer(out_f, in_f, 5)
+    x = torch.randn(rows, in_f, generator=torch.Generator().manual_seed(6)).bfloat16().cuda()
+    plain = layer(x)
+    at = 70 % in_f
+    bad = x.clone()
+    bad[0, at], bad[1, at] = float("inf"), 3e38         # one value: 3e38 w is finite, 3e38 (16 + code) is not
+    if rows > 5:
+        bad[3, 1], bad[3, in_f - 1], bad[4, at], bad[rows - 1, 9] = float("inf"), float("inf"), float("-inf"), float("nan")
+    got, want = layer(bad).double(), bad.double() @ layer.weight.double().t()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(want)) and torch.isinf(got[0]).any()
+    fin = torch.isfinite(want[1])
+    # 3e38 times a weight rounded to bf16 (2^-9 of it) or not, and the output's own rounding
+    assert fin.all() and ((got[1] - want[1]).abs() <= 2.0 ** -7 * want[1].abs() + 2.0 ** -20 * 3e38).all()
+    same = [r for r in range(rows) if bool((bad[r] == x[r]).all())]
+    assert torch.equal(got[same], plain[same].double())
+
+
+def test_silu_infinities():
+    gate_up = _layer(200, 512, 7)
+    x = torch.randn(4, 512, generator=torch.Generator().manual_seed(8)).bfloat16().cuda()
+    x[0, 3], x[2, 500] = float("inf"), float("-inf")
+    gu = F.linear(x, gate_up.weight)
+    want, got = F.silu(gu[:, :100]) * gu[:, 100:], q4_rows_silu(x, gate_up)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))

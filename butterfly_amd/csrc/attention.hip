@@ -1538,6 +1538,11 @@ static PageArgs page_args(const AttnArgs& a) {
   return g;
 }
 
+// Whether a paged streaming batch runs on win_attn_kernel.
+static bool stream_on_win(int64_t window, int bs, int kcap, float scale) {
+  return win_path(window, chunk_blocks_max(bs) * (int64_t)kcap, scale, 0, 1);
+}
+
 // One attention launch: the MFMA kernel where its conditions hold, else the paged MFMA kernel
 // (bf16), the fp32 tile kernel or the generic one.
 static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, const char* what) {
@@ -1696,7 +1701,7 @@ static int launch_attention_batch(const AttnArgs* ch, const void* const* kin, co
       pb.upd_wgs = ux * upd_rows * 2;
     }
     BFLY_CHECK_ARG(nch_max * n * groups * (a.hq / a.hkv) + pb.upd_wgs < (1 << 30), "%s: grid too large", what);
-    if (win_path(a.W, chunk_blocks_max(a.bs) * (int64_t)a.kcap, a.scale, 0, 1))
+    if (stream_on_win(a.W, a.bs, a.kcap, a.scale))
       launch_win_batch(page_args(a), pb, a.d, (int)nch_max, stream);
     else
       launch_page_batch(page_args(a), pb, a.d, (int)nch_max, stream);
@@ -1836,9 +1841,9 @@ extern "C" int bfly_attend_cache(const void* q, int dtype, int64_t batch, int hq
 // per-chunk path.  Chunk c's attention and chunk c+1's update share one launch
 // when they touch disjoint ring slots and pool rows: the update writes positions
 // [P, P + len_{c+1}) (P = end of chunk c) and pool rows >= the summaries chunk c
-// reads, while chunk c's attention reads pages no lower than P - len_c - halo
-// (halo = the window's whole pages and one more), so len_c + len_{c+1} + halo <= ring
-// capacity keeps them apart.
+// reads, while chunk c's attention reads rows no lower than P - len_c - halo (stream_halo: the
+// whole pages that its kernel stages), so len_c + len_{c+1} + halo <= ring capacity keeps
+// them apart.
 namespace {
 
 struct StreamCounters {
@@ -1974,7 +1979,10 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
     bool from_inputs = false;   // the attention reads the batch's own tokens from the chunk inputs
     int stop_rc = BFLY_OK;   // the chunk after the batch does not fit (its error)
   };
-  const int64_t halo = (window - 1 + kPage - 1) / kPage * kPage + kPage;
+  const StreamKernel kernel = mfma_ok ? StreamKernel::kMfma
+                              : stream_on_win(window, block_size, kcap, scale) ? StreamKernel::kWindow
+                                                                               : StreamKernel::kPaged;
+  const int64_t halo = stream_halo(kernel, window);
   const int64_t budget = (ring_capacity - halo) / 2;
   // Wide batches leave the tokens below their tail out of the ring; the call's last launch copies
   // those that its last ring_capacity positions hold (copy_rest), so that the whole ring is what one
@@ -1999,9 +2007,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
     StreamCounters st = s0;
     int64_t blocks = 0, total_len = 0, count = 0, take = 0;
     bool from_inputs = true;
-    // (the W <= 64 kernel stages the whole page before the queries' own)
-    const int64_t reach = window - 1 > kPage ? window - 1 : kPage;
-    const int64_t ring_lo = s0.offset > reach ? (s0.offset - reach) / kPage * kPage : 0;
+    const int64_t ring_lo = stream_ring_lo(kernel, s0.offset, window);
     for (int64_t c = from; c < n_chunks && count < kMaxUpdateParts; ++c) {
       const int64_t len = chunk_len[c];
       StreamCounters nx = st;
@@ -2071,7 +2077,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // Whether `nx`'s update may run beside `cur`'s attention: by length, or because the attention reads
   // only its halo from the ring and the update's appended tokens take other slots.
   auto fuses = [&](const Batch& cur, const Batch& nx) {
-    return cur.total + nx.total + halo <= ring_capacity ||
+    return stream_apart(cur.total, nx.total, halo, ring_capacity) ||
            (wide && cur.from_inputs && ring_disjoint(nx.job.offset + nx.job.append_from, nx.job.offset + nx.total, cur.ring_lo,
                                              cur.job.offset, ring_capacity));
   };

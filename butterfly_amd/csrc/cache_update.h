@@ -14,6 +14,7 @@
 #pragma once
 
 #include "bfly_common.h"
+#include "stream_plan.h"
 
 namespace bfly {
 
@@ -224,14 +225,6 @@ __device__ __forceinline__ void cache_update_body(const UpdateJob& u, int64_t bx
     return ring_row(tok);
   };
   pool_rows<T, VEC, 16>(tok_ptr, (int64_t)u.bs, dst, d, part, t);
-}
-
-// Whether positions [w_lo, w_hi) and the earlier positions [r_lo, r_hi) (r_hi <= w_lo) share no ring
-// slot: no difference w - r is a multiple of the ring.
-inline bool ring_disjoint(int64_t w_lo, int64_t w_hi, int64_t r_lo, int64_t r_hi, int64_t ring) {
-  if (w_lo >= w_hi || r_lo >= r_hi) return true;
-  const int64_t least = w_lo - (r_hi - 1), most = w_hi - 1 - r_lo;
-  return (least - 1) / ring == most / ring;
 }
 
 // One bf16 update job in one launch (compress.hip); rows = batch x kv heads.

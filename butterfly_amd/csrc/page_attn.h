@@ -298,9 +298,10 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
 
   page_u32x4 kst[LD], vst[LD];
   int cand[LD];      // kRouted: the staged rows' list entries
-  // Loads are unconditional: row 0 stands in for a row that does not exist.  Such a row is masked
-  // in the scores, and no value of it is needed (its V takes weight 0; were it infinite, the page
-  // would be summed key by key), so nothing waits for the loads before the page is stored.
+  // Loads are unconditional: the page's nearest position that exists (a window page has one) or summary row 0
+  // stands in for a row that does not.  Such a row is masked in the scores, and no value of it is needed (its
+  // V takes weight 0; were it infinite, the page would be summed key by key), so nothing waits for the loads
+  // before the page is stored.
   auto fetch = [&](int it) {
     int rr[LD];
     const __bf16 *kr = ksb, *vr = vsb;
@@ -323,11 +324,10 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
       }
 #pragma unroll
       for (int j = 0; j < LD; ++j) {
-        const int r = (tid + j * NTHR) / C::PIECES;
-        const bool ok = p0 + r >= a.key_lo && p0 + r < a.kv_len;
+        const int r = min(max((tid + j * NTHR) / C::PIECES, a.key_lo - p0), a.kv_len - 1 - p0);
         int x = r0 + r;
         if (wrap && x >= wrap) x -= wrap;
-        rr[j] = ok ? x : 0;
+        rr[j] = x;
       }
     } else if constexpr (MODE == kPageFused) {
 #pragma unroll

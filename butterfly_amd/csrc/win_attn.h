@@ -409,7 +409,7 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
 
 // Whether win_attn_kernel takes a launch that page_attn_kernel takes: 64 < W <= 128 (a shorter window
 // wastes most of its nine tiles), summaries in one tile, rows to stand in for those that do not
-// exist, a ring that the staged rows do not wrap twice.
+// exist.
 static inline bool win_path(int64_t W, int64_t slots, float scale, int64_t key_lo, int64_t kv_len) {
   return W > 64 && W <= kWinMax && slots <= kWinSlots && scale > 0.f && key_lo < kv_len;
 }

@@ -252,3 +252,28 @@ def test_stream_batches_match_single_chunks(case):
     if w > 64 or min(a + b for a, b in zip(lens[1:], lens[2:])) > (x.tail_capacity - 128) // 2:
         assert torch.equal(x.ring_state().ring_k, y.ring_state().ring_k)
         assert torch.equal(x.ring_state().ring_v, y.ring_state().ring_v)
+
+
+@pytest.mark.parametrize("w,cw,d,bs", [(1, 64, 64, 64), (65, 96, 128, 128), (65, 65, 64, 64), (40, 64, 128, 32)])
+def test_streams_off_the_grid_keep_infinities_with_their_rows(w, cw, d, bs):
+    """Chunks off the page grid through the native loop (each update beside the attention before it) against one
+    core call per chunk, with infinities and NaN among the values: the staged rows that every query masks, down
+    to three pages below a chunk, are none that the update beside writes."""
+    hq, hkv, lens = 4, 2, [100] + [37, 90, 64, 11, 130, 75] * 8
+    cfg = bf.compressed_butterfly_config(block_size=bs, compressed_local_window_tokens=w, block_partner_rule="xor")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    chunks = [tuple(torch.randn(1, h, n, d, generator=g, device="cuda").bfloat16() for h in (hq, hkv, hkv)) for n in lens]
+    for i in range(3, len(chunks), 5):
+        chunks[i][2][0, 0, 3, 1], chunks[i][2][0, 1, 7, d - 1] = math.inf, math.nan
+    caches = [bf.CompressedKVCache(block_size=bs, local_window_tokens=cw, max_kv_size=sum(lens), max_chunk_size=130)
+              for _ in range(2)]
+    core = bf.ButterflyAttentionCore(cfg, 2)
+    got = bf.chunked_prefill(core, chunks, caches[0])
+    assert core.last_profile.notes.get("native_chunk_loop")
+    for i, c in enumerate(chunks):
+        a, b = got[i].float(), core(*c, caches[1]).float()
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b)), i
+        fin = torch.isfinite(b)
+        assert ((a - b)[fin].abs() <= 2 * BF16_ROUNDING * b[fin].abs() + 2 * ABS).all(), i
+    for a, b in zip(caches[0].get_compressed_state()[:4], caches[1].get_compressed_state()[:4]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))

@@ -42,6 +42,11 @@ from typing import Callable, List, Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch import _C
+from torch.autograd import forward_ad
+from torch.compiler import is_compiling
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _native
 from ._device import on, stream_of
@@ -210,20 +215,39 @@ def q4_gemv_silu(x: torch.Tensor, gate_up: QuantLinear) -> torch.Tensor:
 
 def q4_rows_fits(x: torch.Tensor, layer: QuantLinear) -> bool:
     """Whether ``x`` holds 2 to 32 bf16 rows that ``bfly_q4_rows`` multiplies from the codes: a plain
-    GPU tensor that no gradient, tangent or transform follows (those see the GEMM), inputs in whole
-    runs of 256, groups of 64.  Measured (8 / 16 / 32 rows, us): 2048 x 3072 4.7 / 5.2 / 7.1 against
-    8.5 for the GEMM over expanded weights, 2048 x 151936 40 / 42 / 100 against 205 / 205 / 150; at 64
-    rows the GEMM is faster, and from 17 rows on for more than 4096 inputs (6144 x 2048, 17 rows:
-    12.6 against 11.7)."""
-    n = layer.in_features
+    GPU tensor in a call that nothing else follows (``_followed``: those see the GEMM), inputs in whole
+    runs of 256, groups of 64.  Measured (8 / 16 / 32 rows,
+    us): 2048 x 3072 4.7 / 5.2 / 7.1 against 8.5 for the GEMM over expanded weights, 2048 x 151936
+    40 / 42 / 100 against 205 / 205 / 150; at 64 rows the GEMM is faster, and from 17 rows on for more
+    than 4096 inputs (6144 x 2048, 17 rows: 12.6 against 11.7)."""
+    b = layer._buffers                     # (attribute access on a module costs more than the tests)
+    packed = b.get("packed")
+    if packed is None:
+        return False
+    n = 2 * packed.shape[1]
     if not 2 * n <= x.numel() <= (16 if n > 4096 else Q4_MAX_ROWS) * n:
         return False
-    if type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.bfloat16 or x.shape[-1] != n \
-            or n % 256 or layer.group != 64 or layer.packed.device != x.device \
-            or (layer.packed.data_ptr() | layer.scale_bias.data_ptr()) % 16:
+    weight, pairs = b.get("weight"), b["scale_bias"]
+    if weight is None or _followed(x, weight):
         return False
-    return not (torch.is_grad_enabled() and x.requires_grad) and torch.autograd.forward_ad._current_level < 0 \
-        and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+    if type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.bfloat16 or x.shape[-1] != n \
+            or n % 256 or layer.group != 64 or packed.device != x.device \
+            or pairs.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
+            or (packed.data_ptr() | pairs.data_ptr()) % 16:
+        return False
+    return True
+
+
+def _followed(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether anything follows the operators of this call, which a native call would hide from it: a gradient of
+    ``x`` or ``weight``, a tangent, a transform, a trace or compilation, a dispatch or function mode (other than a
+    default device), autocast."""
+    return (is_compiling() or _C._get_tracing_state() is not None
+            or ((x.requires_grad or weight.requires_grad) and torch.is_grad_enabled())
+            or forward_ad._current_level >= 0 or _C._functorch.is_functorch_wrapped_tensor(x)
+            or _C._len_torch_dispatch_stack() > 0 or torch.is_autocast_enabled()
+            or (_C._len_torch_function_stack() > 0
+                and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())))
 
 
 def _rows16(x: torch.Tensor) -> torch.Tensor:
@@ -234,23 +258,23 @@ def _rows16(x: torch.Tensor) -> torch.Tensor:
 
 def q4_rows(x: torch.Tensor, layer: QuantLinear) -> torch.Tensor:
     """``layer(x)`` for 2 to 32 rows (``q4_rows_fits``) through ``bfly_q4_rows``."""
-    xr = _rows16(x)
-    out = torch.empty(*x.shape[:-1], layer.out_features, dtype=torch.bfloat16, device=x.device)
-    with on(x.device):
-        _native.call("bfly_q4_rows", xr.data_ptr(), xr.shape[0], layer.packed.data_ptr(), layer.scale_bias.data_ptr(),
-                     layer.out_features, layer.in_features, layer.group, out.data_ptr(), stream_of(x))
+    xr, packed, dev = _rows16(x), layer.packed, x.device
+    f, half = packed.shape
+    out = torch.empty(*x.shape[:-1], f, dtype=torch.bfloat16, device=dev)
+    with on(dev):
+        _native.call("bfly_q4_rows", xr.data_ptr(), xr.shape[0], packed.data_ptr(), layer.scale_bias.data_ptr(),
+                     f, 2 * half, layer.group, out.data_ptr(), stream_of(dev))
     return out
 
 
 def q4_rows_silu(x: torch.Tensor, gate_up: QuantLinear) -> torch.Tensor:
     """``SiLU(gate(x)) * up(x)`` for 2 to 32 rows (``q4_rows_fits``) through ``bfly_q4_rows_silu``."""
-    xr = _rows16(x)
-    f = gate_up.out_features // 2
-    out = torch.empty(*x.shape[:-1], f, dtype=torch.bfloat16, device=x.device)
-    with on(x.device):
-        _native.call("bfly_q4_rows_silu", xr.data_ptr(), xr.shape[0], gate_up.packed.data_ptr(),
-                     gate_up.scale_bias.data_ptr(), f, gate_up.in_features, gate_up.group, f, out.data_ptr(),
-                     stream_of(x))
+    xr, packed, dev = _rows16(x), gate_up.packed, x.device
+    f, half = packed.shape[0] // 2, packed.shape[1]
+    out = torch.empty(*x.shape[:-1], f, dtype=torch.bfloat16, device=dev)
+    with on(dev):
+        _native.call("bfly_q4_rows_silu", xr.data_ptr(), xr.shape[0], packed.data_ptr(),
+                     gate_up.scale_bias.data_ptr(), f, 2 * half, gate_up.group, f, out.data_ptr(), stream_of(dev))
     return out
 
 

@@ -125,3 +125,27 @@ def test_silu_infinities():
     gu = F.linear(x, gate_up.weight)
     want, got = F.silu(gu[:, :100]) * gu[:, 100:], q4_rows_silu(x, gate_up)
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+
+
+def _few(layer, n=4):
+    return torch.randn(n, layer.in_features, generator=torch.Generator().manual_seed(9)).bfloat16().cuda()
+
+
+def test_traced_layers_record_the_product():
+    layer = _layer(48, 256, 11)
+    x = _few(layer)
+    traced = torch.jit.trace(layer, (x,), check_trace=False)
+    other = torch.flip(x, (0,))
+    assert torch.equal(traced(other), F.linear(other, layer.weight))
+
+
+def test_weight_gradients_and_autocast():
+    layer = _layer(48, 256, 12)
+    x = _few(layer)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert layer(x).dtype == torch.float16
+    layer.weight.requires_grad_()
+    layer(x).float().sum().backward()
+    assert torch.allclose(layer.weight.grad.float(), x.float().sum(0).expand(48, -1), rtol=2 ** -7, atol=1e-3)
+    layer.weight.requires_grad_(False)
+    assert q4_rows_fits(x, layer)

@@ -250,6 +250,16 @@ def _followed(x: torch.Tensor, weight: torch.Tensor) -> bool:
                 and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())))
 
 
+def _hooked(layer: nn.Module) -> bool:
+    """Whether calling ``layer`` runs more than ``QuantLinear.forward``: hooks of its own or of all modules, another
+    class or a forward set on the instance."""
+    m = torch.nn.modules.module
+    return (type(layer) is not QuantLinear or "forward" in layer.__dict__
+            or bool(layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks
+                    or layer._backward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks
+                    or m._global_backward_hooks or m._global_backward_pre_hooks))
+
+
 def _rows16(x: torch.Tensor) -> torch.Tensor:
     """``x`` as a contiguous, 16-byte aligned [rows, in] tensor."""
     x = x.reshape(-1, x.shape[-1])
@@ -666,7 +676,7 @@ class MLP(nn.Module):
         if x.numel() <= Q4_MAX_ROWS * x.shape[-1]:
             if _one_row(x) and self.gate_up.gemv_from_codes:
                 return self.down_proj(q4_gemv_silu(x, self.gate_up))
-            if q4_rows_fits(x, self.gate_up):
+            if not _hooked(self.gate_up) and q4_rows_fits(x, self.gate_up):
                 return self.down_proj(q4_rows_silu(x, self.gate_up))
         if _hip(x):
             gu = self.gate_up(x)                           # [..., 2f]: gate columns, then up columns

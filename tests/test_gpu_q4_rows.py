@@ -149,3 +149,15 @@ def test_weight_gradients_and_autocast():
     assert torch.allclose(layer.weight.grad.float(), x.float().sum(0).expand(48, -1), rtol=2 ** -7, atol=1e-3)
     layer.weight.requires_grad_(False)
     assert q4_rows_fits(x, layer)
+
+
+def test_mlp_hooks_fire():
+    cfg = DecoderConfig(hidden_size=512, intermediate_size=1024)
+    mlp = MLP(cfg, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda")
+    x, seen = torch.randn(6, 1, 512, device="cuda").bfloat16(), []
+    plain = mlp(x)
+    handle = mlp.gate_up.register_forward_hook(lambda m, a, out: seen.append(out.shape))
+    got = mlp(x)
+    handle.remove()
+    assert seen == [(6, 1, 2048)]
+    assert ((got - plain).float().norm() / plain.float().norm()).item() <= 2 ** -8

@@ -8,7 +8,7 @@ from torch.fx.experimental.proxy_tensor import make_fx
 from torch.overrides import TorchFunctionMode
 from torch.utils.flop_counter import FlopCounterMode
 
-from butterfly_amd.decoder import QuantLinear, _followed
+from butterfly_amd.decoder import QuantLinear, _followed, _hooked
 
 
 def _layer(out_f=6, in_f=128, seed=0):
@@ -66,3 +66,25 @@ def test_compiled_layers_see_the_product():
     layer = _layer()
     got = torch.compile(layer, backend="eager", fullgraph=True)(X)
     assert torch.equal(got, F.linear(X, layer.weight))
+
+
+def test_hooks_and_wrappers():
+    layer = _layer()
+    assert not _hooked(layer)
+    for register in (layer.register_forward_hook, layer.register_forward_pre_hook,
+                     torch.nn.modules.module.register_module_forward_hook,
+                     torch.nn.modules.module.register_module_forward_pre_hook):
+        handle = register(lambda *a: None)
+        assert _hooked(layer)
+        handle.remove()
+        assert not _hooked(layer)
+    handle = layer.register_full_backward_hook(lambda *a: None)
+    assert _hooked(layer)
+    handle.remove()
+
+    class Wrapped(QuantLinear):
+        pass
+
+    assert _hooked(Wrapped(128, 4))
+    layer.forward = lambda x: x
+    assert _hooked(layer)

@@ -105,7 +105,12 @@ class QuantLinear(nn.Module):
     Buffers: ``packed`` (two codes per byte, low nibble first), ``scale`` and ``bias``
     (bf16 per group), ``scale_bias`` (the same pairs interleaved, [out, in/group, 2], the
     layout ``bfly_q4_gemv`` reads) and ``weight`` (dequantized once to bf16, for the
-    multi-row GEMMs and for CPU copies of the model)."""
+    multi-row GEMMs and for CPU copies of the model).
+
+    ``codes_hold`` tells whether ``weight`` still is what the codes say.  An edit in place, a new
+    tensor in a buffer's place or a load of other values ends that, and products of two rows and
+    more then follow ``weight`` (an edit through ``weight.data``, which PyTorch does not count, is
+    not seen by products of 2 to 32 rows)."""
 
     def __init__(self, in_features: int, out_features: int, *, generator: Optional[torch.Generator] = None,
                  device=None, group: int = 64, weight: Optional[torch.Tensor] = None):
@@ -116,11 +121,59 @@ class QuantLinear(nn.Module):
         self._set(*quantize_affine(weight, group))
 
     def _set(self, packed, scale, bias):
-        self.register_buffer("packed", packed)
-        self.register_buffer("scale", scale)
-        self.register_buffer("bias", bias)
-        self.register_buffer("scale_bias", torch.stack([scale, bias], -1).contiguous())
-        self.register_buffer("weight", dequantize_affine(packed, scale, bias, self.group))
+        with torch.inference_mode(False):      # (an inference tensor does not count its edits)
+            self.register_buffer("packed", packed.clone() if packed.is_inference() else packed)
+            self.register_buffer("scale", scale)
+            self.register_buffer("bias", bias)
+            self.register_buffer("scale_bias", torch.stack([scale, bias], -1).contiguous())
+            self.register_buffer("weight", dequantize_affine(packed, scale, bias, self.group))
+        self._bind()
+
+    # the buffers that the codes' products depend on and their edit counts while ``weight`` matched the codes
+    _bound = None
+
+    def _bind(self) -> None:
+        b = self._buffers
+        ts = (b["weight"], b["packed"], b["scale_bias"])
+        self._bound = None if any(type(t) is not torch.Tensor or t.is_inference() for t in ts) else \
+            (*ts, *(t._version for t in ts), ts[0].data_ptr())
+
+    def codes_hold(self) -> bool:
+        """Whether ``weight`` is known to be ``codes * scale + bias`` (see the class)."""
+        m, b = self._bound, self._buffers
+        return (m is not None and b.get("weight") is m[0] and b["packed"] is m[1] and b["scale_bias"] is m[2]
+                and m[0]._version == m[3] and m[1]._version == m[4] and m[2]._version == m[5]
+                and m[0].data_ptr() == m[6])
+
+    def _apply(self, fn, recurse=True):
+        held = self.codes_hold()
+        super()._apply(fn, recurse)
+        if held:
+            self._bind()
+        return self
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        super()._load_from_state_dict(*args, **kwargs)
+        if not self.codes_hold() and self._weight_matches():
+            self._bind()
+
+    def _weight_matches(self) -> bool:
+        """The comparison itself, a slice of rows at a time: what ``codes_hold`` says after a load."""
+        packed, scale, bias, pairs, weight = ts = [self._buffers.get(name) for name in _Q4_TENSORS]
+        if any(type(t) is not torch.Tensor or t.is_meta or t.device != packed.device for t in ts) or \
+                any(t.dtype != torch.bfloat16 for t in ts[1:]) or torch._C._len_torch_dispatch_stack() > 0:
+            return False
+        return all(torch.equal(torch.stack([scale[r], bias[r]], -1), pairs[r])
+                   and torch.equal(dequantize_affine(packed[r], scale[r], bias[r], self.group), weight[r])
+                   for r in (slice(at, at + 16384) for at in range(0, packed.shape[0], 16384)))
+
+    def __getstate__(self):
+        return {**self.__dict__, "_bound": self.codes_hold()}
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        if self.__dict__.pop("_bound", False):
+            self._bind()
 
     @property
     def in_features(self) -> int:
@@ -137,14 +190,20 @@ class QuantLinear(nn.Module):
         fused = cls.__new__(cls)
         nn.Module.__init__(fused)
         fused.group = parts[0].group
-        for name in _Q4_TENSORS:
-            fused.register_buffer(name, torch.cat([getattr(m, name) for m in parts]))
+        held = all(m.codes_hold() for m in parts)
+        with torch.inference_mode(False):
+            for name in _Q4_TENSORS:
+                fused.register_buffer(name, torch.cat([getattr(m, name) for m in parts]))
         row = 0
         for m in parts:
             n = m.out_features
             for name in _Q4_TENSORS:
                 setattr(m, name, getattr(fused, name)[row:row + n])
             row += n
+        for m in (fused, *parts):
+            m._bound = None
+            if held:
+                m._bind()
         return fused
 
     @property
@@ -216,7 +275,7 @@ def q4_gemv_silu(x: torch.Tensor, gate_up: QuantLinear) -> torch.Tensor:
 def q4_rows_fits(x: torch.Tensor, layer: QuantLinear) -> bool:
     """Whether ``x`` holds 2 to 32 bf16 rows that ``bfly_q4_rows`` multiplies from the codes: a plain
     GPU tensor in a call that nothing else follows (``_followed``: those see the GEMM), inputs in whole
-    runs of 256, groups of 64.  Measured (8 / 16 / 32 rows,
+    runs of 256, groups of 64, a weight that is still the codes' own.  Measured (8 / 16 / 32 rows,
     us): 2048 x 3072 4.7 / 5.2 / 7.1 against 8.5 for the GEMM over expanded weights, 2048 x 151936
     40 / 42 / 100 against 205 / 205 / 150; at 64 rows the GEMM is faster, and from 17 rows on for more
     than 4096 inputs (6144 x 2048, 17 rows: 12.6 against 11.7)."""
@@ -235,7 +294,7 @@ def q4_rows_fits(x: torch.Tensor, layer: QuantLinear) -> bool:
             or pairs.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
             or (packed.data_ptr() | pairs.data_ptr()) % 16:
         return False
-    return True
+    return layer.codes_hold()
 
 
 def _followed(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -756,8 +815,9 @@ class Decoder(nn.Module):
         else embed @ h^T over the dequantized table."""
         if _one_row(h) and self.lm_head.gemv_from_codes:
             return q4_gemv(h, self.lm_head)
-        if q4_rows_fits(h, self.lm_head):
-            return q4_rows(h, self.lm_head)
+        e = self.embed_tokens
+        if not e.requires_grad and q4_rows_fits(h, self.lm_head) and e.data_ptr() == self.lm_head.weight.data_ptr():
+            return q4_rows(h, self.lm_head)      # (embed_tokens is lm_head.weight: one storage, one edit count)
         return torch.matmul(self.embed_tokens, h.t()).t()
 
     def _rope(self, start: int, t: int, device):

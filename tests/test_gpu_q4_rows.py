@@ -12,7 +12,7 @@ import torch.nn.functional as F
 
 from butterfly_amd import _native
 from butterfly_amd._device import stream_of
-from butterfly_amd.decoder import MLP, DecoderConfig, QuantLinear, q4_rows, q4_rows_fits, q4_rows_silu
+from butterfly_amd.decoder import MLP, Decoder, DecoderConfig, QuantLinear, q4_rows, q4_rows_fits, q4_rows_silu
 
 pytestmark = pytest.mark.gpu
 
@@ -139,7 +139,7 @@ def test_traced_layers_record_the_product():
     assert torch.equal(traced(other), F.linear(other, layer.weight))
 
 
-def test_weight_gradients_and_autocast():
+def test_weight_gradients_edits_and_autocast():
     layer = _layer(48, 256, 12)
     x = _few(layer)
     with torch.autocast("cuda", dtype=torch.float16):
@@ -149,6 +149,8 @@ def test_weight_gradients_and_autocast():
     assert torch.allclose(layer.weight.grad.float(), x.float().sum(0).expand(48, -1), rtol=2 ** -7, atol=1e-3)
     layer.weight.requires_grad_(False)
     assert q4_rows_fits(x, layer)
+    layer.weight[7].zero_()
+    assert (layer(x)[:, 7] == 0).all() and torch.equal(layer(x), F.linear(x, layer.weight))
 
 
 def test_mlp_hooks_fire():
@@ -161,3 +163,14 @@ def test_mlp_hooks_fire():
     handle.remove()
     assert seen == [(6, 1, 2048)]
     assert ((got - plain).float().norm() / plain.float().norm()).item() <= 2 ** -8
+
+
+def test_logits_follow_the_embedding():
+    cfg = DecoderConfig(vocab_size=512, hidden_size=256, num_layers=0)
+    model = Decoder(cfg, device="cuda")
+    h = torch.randn(4, 256, device="cuda").bfloat16()
+    before = model._logits(h)
+    with torch.no_grad():
+        model.embed_tokens[5].zero_()
+    after = model._logits(h)
+    assert (after[:, 5] == 0).all() and ((after - before)[:, :5].float().abs() <= 2 ** -6 * before[:, :5].float().abs() + 1e-2).all()

@@ -1644,6 +1644,53 @@ static int launch_attention(const AttnArgs& a, int dtype, hipStream_t stream, co
   return BFLY_OK;
 }
 
+// The attention of a batch of streaming chunks (cb.c[0 .. nch), cb.upd and its item counts filled) and,
+// with upd_wgs > 0, the next batch's cache update on workgroups behind them.
+static void launch_page_batch(PageArgs a, PageBatch cb, int d, int nchunks_max, hipStream_t stream) {
+  const int gsz = a.hq / a.hkv;
+  auto go = [&](auto kernel, int heads, int nh) {
+    a.c_first = 0;
+    a.nchunks = nchunks_max;
+    a.nparts = (gsz + heads - 1) / heads;
+    a.items = nchunks_max * cb.nch * a.batch * a.hkv * a.nparts;
+    a.per_xcd = (a.items + 7) / 8;
+    cb.attn_blocks = 8 * a.per_xcd;
+    const int64_t extra = (cb.upd_wgs + nh - 1) / nh;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(cb.attn_blocks + extra)), dim3(256 * nh), 0, stream, a, cb);
+  };
+  if (d == 256) go(page_attn_kernel<256, 1, 2, kPageFused, true>, 2, 2);
+  else if (d == 128 && gsz > 1) go(page_attn_kernel<128, 2, 1, kPageFused, true>, 2, 1);
+  else if (d == 128) go(page_attn_kernel<128, 1, 1, kPageFused, true>, 1, 1);
+  else if (gsz > 1) go(page_attn_kernel<64, 2, 1, kPageFused, true>, 2, 1);
+  else go(page_attn_kernel<64, 1, 1, kPageFused, true>, 1, 1);
+}
+
+// launch_page_batch on win_attn_kernel.
+static void launch_win_batch(PageArgs a, PageBatch cb, int d, int nchunks_max, hipStream_t stream) {
+  const int gsz = a.hq / a.hkv;
+  auto go = [&](auto kernel, int heads, int nh) {
+    a.c_first = 0;
+    a.nchunks = nchunks_max;
+    a.nparts = (gsz + heads - 1) / heads;
+    a.items = nchunks_max * cb.nch * a.batch * a.hkv * a.nparts;
+    a.per_xcd = (a.items + 7) / 8;
+    cb.attn_blocks = 8 * a.per_xcd;
+    const int64_t extra = (cb.upd_wgs + nh - 1) / nh;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(cb.attn_blocks + extra)), dim3(256 * nh), 0, stream, a, cb);
+  };
+  const int64_t units = (int64_t)nchunks_max * cb.nch * a.batch * a.hkv;
+  if (d == 256) {
+    if (gsz >= 3 && units * ((gsz + 3) / 4) >= 128) go(win_attn_kernel<256, 2, 2, kPageFused, true>, 4, 2);
+    else go(win_attn_kernel<256, 1, 2, kPageFused, true>, 2, 2);
+  } else if (d == 128) {
+    if (gsz > 1) go(win_attn_kernel<128, 2, 1, kPageFused, true>, 2, 1);
+    else go(win_attn_kernel<128, 1, 1, kPageFused, true>, 1, 1);
+  } else {
+    if (gsz > 1) go(win_attn_kernel<64, 2, 1, kPageFused, true>, 2, 1);
+    else go(win_attn_kernel<64, 1, 1, kPageFused, true>, 1, 1);
+  }
+}
+
 // The attention of n (<= kMaxUpdateParts) consecutive streaming chunks in one launch (neighbour
 // rows from each chunk's topology; `paged`: the paged kernel, for what the W <= 64 one does not
 // take): ch[j] holds chunk j's arguments as

@@ -2100,7 +2100,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
         (void)frc;
         break;
       }
-      if (!from_inputs && total_len > budget) break;   // no longer prefix can fit
+      if (!(wide && from_inputs) && total_len > budget) break;   // no longer prefix can fit
     }
     if (take < count) bt.stop_rc = BFLY_OK;            // the batch ends before the chunk that did not fit
     bt.count = take;
@@ -2129,11 +2129,16 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
                                              cur.job.offset, ring_capacity));
   };
   auto launch_update = [&](const UpdateJob& j) -> int { return launch_update_job(j, rows, stream); };
-  // the tokens of chunks [0, done) below the tail that st leaves, of the last ring_capacity positions
+  // the tokens of chunks [0, done) below the tail that st leaves, of the last ring_capacity positions, where
+  // a batch left any of those out (left_out: the end of the last such tokens)
+  int64_t left_out = 0;
+  auto note_left_out = [&](const UpdateJob& j) {
+    if (j.append_from > 0) left_out = j.offset + j.append_from;
+  };
   auto copy_rest = [&](const StreamCounters& st, int64_t done) -> int {
     const int64_t hi = st.offset - st.tail;
     int64_t lo = st.offset - ring_capacity, pos = call_offset, c = 0;
-    if (!wide || lo >= hi) return BFLY_OK;
+    if (!wide || lo >= hi || left_out <= lo) return BFLY_OK;
     while (c < done && pos < hi) {
       UpdateJob j{};
       j.ring_k = ring_k; j.ring_v = ring_v; j.pool_k = pool_k; j.pool_v = pool_v;
@@ -2169,6 +2174,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   if (cur.count == 0) return cur.stop_rc;
   rc = launch_update(cur.job);
   if (rc) return rc;
+  note_left_out(cur.job);
   s = cur.end;
   publish(s);
   if (cur.overflow) return BFLY_ERR_CAPACITY;   // the message was set when it was planned
@@ -2200,6 +2206,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
       return rc ? rc : nxt.stop_rc;
     }
     s = nxt.end;
+    note_left_out(nxt.job);
     publish(s);
     if (nxt.overflow) {
       rc = copy_rest(s, next_from + nxt.count);

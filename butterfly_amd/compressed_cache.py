@@ -427,9 +427,10 @@ class CompressedKVCache:
                  and (d in (64, 128) or (d == 256 and q.dtype == torch.bfloat16)))
         if fused and w > 64:
             # the general path has fewer conditions: a first step (no buffers yet), other shapes than the
-            # keys' and a cache that pools the newest block go there
+            # keys' (also those that it refuses, with the token appended) and a cache that pools the newest
+            # block go there
             fused = (self._ring_k is not None and self.local_window_tokens > 0 and q.shape[0] == keys.shape[0]
-                     and d == keys.shape[3] == values.shape[3]
+                     and d == keys.shape[3] == values.shape[3] and q.shape[1] % keys.shape[1] == 0
                      and decode_wide_fits((q, self._ring_k, self._ring_v, self._pool_k, self._pool_v),
                                           rows=self.tail_capacity, ring_capacity=self.tail_capacity,
                                           kv_len=self.offset + 1, pool_rows=self.summary_capacity,

@@ -100,6 +100,25 @@ def test_general_path_calls_stay_accepted():
         assert torch.isfinite(out).all()
 
 
+def test_heads_that_do_not_group_are_refused_after_the_append():
+    """Three query heads over two: refused, and the token is in the cache, as on the general path."""
+    k = _rand(6, 1, 2, 301, 64)
+    lay = bf.build_block_butterfly_layout(seq_len=301, block_size=64, num_key_value_heads=2, num_key_value_groups=2,
+                                          layer_idx=0, local_window_blocks=1, sink_count=1, partner_count=1,
+                                          partner_rule="xor")
+    caches = []
+    for w in (100, 129):      # the fused step's windows, the general path's
+        cache = bf.CompressedKVCache(block_size=64, local_window_tokens=128, max_kv_size=400)
+        cache.update(k[:, :, :300].cuda(), k[:, :, :300].cuda())
+        with pytest.raises(ValueError, match="head"):
+            cache.update_and_attend(_rand(7, 1, 3, 1, 64).cuda(), k[:, :, 300:].cuda(), k[:, :, 300:].cuda(), layout=lay,
+                                    local_window_tokens=w)
+        caches.append(cache)
+    for a, b in zip(caches[0].get_compressed_state()[:4], caches[1].get_compressed_state()[:4]):
+        assert torch.equal(a, b)
+    assert caches[0].offset == caches[1].offset == 301
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_weights_keep_fp32_precision(d):
     """Values that cancel under the weights leave the weights' own error: four window rows of each column are

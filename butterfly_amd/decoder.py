@@ -542,10 +542,10 @@ class RopeTable:
 
     def fits(self, x: torch.Tensor, d: int) -> bool:
         """Whether a kernel can read its row of the tables by itself: one int64 position, plain fp32 tables of
-        ``d`` columns on ``x``'s device.  Two row selections and their launches less for each layer: a step of
+        ``d`` columns on ``x``'s device, ``rows`` as it stands above.  Two row selections and their launches less for each layer: a step of
         eight sequences through four layers is 214 us so, 231 with the selections."""
         tabs, pos = (self.cos_tab, self.sin_tab), self.pos
-        return (pos.dtype == torch.int64 and pos.numel() == 1 and pos.device == x.device
+        return (type(self).rows is RopeTable.rows and "rows" not in self.__dict__ and pos.dtype == torch.int64 and pos.numel() == 1 and pos.device == x.device
                 and tabs[0].shape == tabs[1].shape
                 and all(t.dtype == torch.float32 and t.ndim == 2 and t.shape[1] == d and t.shape[0] > 0
                         and t.is_contiguous() and t.device == x.device for t in tabs))

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import butterfly_amd as bf
-from butterfly_amd.decoder import Decoder, DecoderConfig, dequantize_affine, quantize_affine
+from butterfly_amd.decoder import Decoder, DecoderConfig, RopeTable, dequantize_affine, quantize_affine
 from oracle.decoder_ref import swap_to_oracle
 
 
@@ -127,3 +127,16 @@ def test_cpu_reference_one_row_products_take_the_gpu_rounding_points():
     assert torch.equal(model.layers[0].mlp.gate_proj(rows), before)  # three rows: the bf16 GEMM
     h = torch.randn(1, 256, generator=g).bfloat16()
     assert torch.equal(model._logits(h), q4_row(h, model.lm_head))
+
+
+def test_rope_tables_with_rows_of_their_own_are_asked_for_them():
+    """A kernel reads its table row by itself only where ``rows`` would give that row."""
+    class Scaled(RopeTable):
+        def rows(self):
+            return tuple(2 * r for r in super().rows())
+
+    tabs, pos, x = (torch.randn(9, 128), torch.randn(9, 128)), torch.tensor([3]), torch.empty(0)
+    assert RopeTable(*tabs, pos).fits(x, 128) and not Scaled(*tabs, pos).fits(x, 128)
+    table = RopeTable(*tabs, pos)
+    table.rows = lambda: tabs
+    assert not table.fits(x, 128)

@@ -21,7 +21,8 @@
 //   * P keeps fp32's worth of precision: it enters the product as two bf16 parts, P = hi + lo up to
 //     2^-17 P, two MFMAs on one V fragment.
 //   * The accumulators are rescaled only when a row's maximum outgrows the reference value by
-//     2^8 (P then stays below 2^8, far inside fp32): a rescale is D / 4 multiplications per head.
+//     2^8 (P then stays below 2^8, far inside fp32), or at all for a page with a V of 2^100 or more (whose
+//     sums would overflow): a rescale is D / 4 multiplications per head.
 //   * A page whose V holds an infinity or NaN goes through plain fp32 sums over the keys each row
 //     attends to (0 * inf in the matrix product would reach rows that do not attend to it).
 //
@@ -109,16 +110,19 @@ __device__ __forceinline__ bf16x8 page_xchg8(bf16x8 v) {
   return __builtin_bit_cast(bf16x8, u);
 }
 
-// Nonzero when any of the 8 bf16 of a piece is an infinity or NaN (all exponent bits set).
-__device__ __forceinline__ bool page_nonfinite(page_u32x4 x) {
+// The largest magnitude of a piece's 8 bf16, its exponent in the upper 8 bits.
+__device__ __forceinline__ unsigned page_magnitude(page_u32x4 x) {
   unsigned t = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const unsigned a = x[i] << 1, b = x[i] << 17;
     t = max(t, max(a, b));
   }
-  return t >= 0xff000000u;
+  return t;
 }
+// From kPageLarge (2^100) on a V is too large for weights of 2^8; kPageNonfinite: an infinity or NaN.
+constexpr unsigned kPageLarge = (127u + 100u) << 24, kPageNonfinite = 0xff000000u;
+__device__ __forceinline__ bool page_nonfinite(page_u32x4 x) { return page_magnitude(x) >= kPageNonfinite; }
 
 // This workgroup's (row, 64-position chunk) item, and in a batch its chunk's arguments put into `a` and its
 // index into zc; false for a workgroup past the items.  Workgroups go round-robin over the 8 XCDs: XCD x
@@ -386,21 +390,23 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
   }
 
   for (int it = 0; it < npages; ++it) {
-    bool bad = false;
+    unsigned worst = 0;
 #pragma unroll
     for (int j = 0; j < LD; ++j) {
       const int i = tid + j * NTHR, r = i / C::PIECES, pc = i % C::PIECES;
       *reinterpret_cast<page_u32x4*>(Ks + r * KP + pc * 8) = kst[j];
       *reinterpret_cast<page_u32x4*>(Vs + r * D + (pc ^ vrow_swizzle<D>(r)) * 8) = vst[j];
-      bad = bad || page_nonfinite(vst[j]);
+      worst = max(worst, page_magnitude(vst[j]));
       if constexpr (MODE == kPageRouted) {
         if (pc == 0) s_n[r] = cand[j];
       }
     }
-    if (bad) s_bad[it & 1] = 1;
+    if (worst >= kPageLarge) atomicMax(&s_bad[it & 1], worst >= kPageNonfinite ? 2 : 1);
     __syncthreads();   // the page is staged
     if (tid == 0) s_bad[(it + 1) & 1] = 0;
-    const bool page_bad = s_bad[it & 1] != 0;
+    const int flag = s_bad[it & 1];
+    const bool page_bad = flag == 2;
+    const float slack = flag != 0 ? 0.f : 8.f;
     if (it + 1 < npages) fetch(it + 1);
 
     const bool win = kWin && it < nwin;
@@ -472,7 +478,7 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
                            fmaxf(fmaxf(s[u][1][0], s[u][1][1]), fmaxf(s[u][1][2], s[u][1][3])));
           mx = col_max4(mx);
           if constexpr (MODE != kPageFused) mtop[u] = fmaxf(mtop[u], mx);
-          if (__any(mx > mref[u] + 8.f)) {
+          if (__any(mx > mref[u] + slack)) {
             const float mn = fmaxf(mref[u], mx);
             const float al = __builtin_amdgcn_exp2f(mref[u] - (mn == -INFINITY ? 0.f : mn));   // 0 at first
             mref[u] = mn;

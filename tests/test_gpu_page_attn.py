@@ -277,3 +277,21 @@ def test_streams_off_the_grid_keep_infinities_with_their_rows(w, cw, d, bs):
         assert ((a - b)[fin].abs() <= 2 * BF16_ROUNDING * b[fin].abs() + 2 * ABS).all(), i
     for a, b in zip(caches[0].get_compressed_state()[:4], caches[1].get_compressed_state()[:4]):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("d,groups", [(64, 1), (128, 2), (128, 4), (256, 2)])
+def test_large_values_stay_finite(d, groups):
+    """Values near bf16's largest under scores that climb by less than the rescaling threshold from group to group:
+    the weighted mean is finite, and no partial sum may overflow on the way."""
+    t, w, bs = 400, 200, 64
+    q = torch.ones(1, groups, t, d).bfloat16()
+    climb = (torch.arange(t) // 32 * 7.6 * math.log(2)) / d ** 0.5      # scores: 7.6 octaves each 32 keys
+    k = climb[None, None, :, None].expand(1, 1, t, d).bfloat16()
+    v = _rand(1, 1, 1, t, d)
+    v[0, 0, 40::50] = 3e36 * v[0, 0, 40::50].sign()
+    scale = d ** -0.5
+    want = oa.swa_stream(q.double(), k.double().expand(1, groups, t, d), v.double().expand(1, groups, t, d), W=w,
+                         scale=scale)[0]
+    got = bf.swa_stream_attention(q.cuda(), k.cuda(), v.cuda(), n_win=w, scale=scale)[0].cpu().double()
+    assert torch.isfinite(got).all()
+    assert ((got - want).norm() / want.norm()).item() <= 2 ** -8

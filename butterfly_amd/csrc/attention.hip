@@ -295,26 +295,6 @@ constexpr int kF32MaxKcap = 16;
 constexpr int f32_win_tiles(int W) { return (W - 1 + 15) / 16 + 1; }   // 5 for 64, 9 for 128
 constexpr int f32_rows(int W) { return 16 * (f32_win_tiles(W) + 1); }
 
-// The three bf16 parts (bit patterns, two per dword, element 0 in the low half) of four floats.
-struct Parts4 {
-  uint2 h, m, l;
-};
-__device__ __forceinline__ Parts4 split_parts(f32x4 x) {
-  uint32_t hb[4], mb[4], lb[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    hb[i] = __float_as_uint(x[i]) & 0xffff0000u;
-    const float rest = x[i] - __uint_as_float(hb[i]);          // exact
-    mb[i] = __float_as_uint(rest) & 0xffff0000u;
-    lb[i] = __float_as_uint(rest - __uint_as_float(mb[i]));     // exact, low 16 bits zero
-  }
-  auto pk = [](uint32_t e0, uint32_t e1) { return (e0 >> 16) | (e1 & 0xffff0000u); };
-  return {{pk(hb[0], hb[1]), pk(hb[2], hb[3])}, {pk(mb[0], mb[1]), pk(mb[2], mb[3])},
-          {pk(lb[0], lb[1]), pk(lb[2], lb[3])}};
-}
-__device__ __forceinline__ bf16x8 join8(uint2 a, uint2 b) {
-  return __builtin_bit_cast(bf16x8, uint4{a.x, a.y, b.x, b.y});
-}
 // c + a b in the six part products (small terms first)
 __device__ __forceinline__ f32x4 mfma_x6(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x4 c) {
   c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], c, 0, 0, 0);

@@ -18,8 +18,8 @@
 // time (two 16-row tiles): S^T = K Q^T, running maximum and sum, O^T += V^T P^T, all on
 // v_mfma_f32_16x16x32_bf16 with fp32 accumulators.  32-key groups without a key for the wave's 16
 // rows are passed over.
-//   * P keeps fp32's worth of precision: it enters the product as two bf16 parts, P = hi + lo up to
-//     2^-17 P, two MFMAs on one V fragment.
+//   * P enters the product whole, all 24 bits of its fp32 value, as three bf16 parts P = hi + mid + lo:
+//     three MFMAs on one V fragment.
 //   * The accumulators are rescaled only when a row's maximum outgrows the reference value by
 //     2^8 (P then stays below 2^8, far inside fp32), or at all for a page with a V of 2^100 or more (whose
 //     sums would overflow): a rescale is D / 4 multiplications per head.
@@ -123,6 +123,28 @@ __device__ __forceinline__ unsigned page_magnitude(page_u32x4 x) {
 // From kPageLarge (2^100) on a V is too large for weights of 2^8; kPageNonfinite: an infinity or NaN.
 constexpr unsigned kPageLarge = (127u + 100u) << 24, kPageNonfinite = 0xff000000u;
 __device__ __forceinline__ bool page_nonfinite(page_u32x4 x) { return page_magnitude(x) >= kPageNonfinite; }
+
+// The three bf16 parts (bit patterns, two per dword, element 0 in the low half) of four floats: together
+// exactly the float, 8 bits of its 24 each.
+struct Parts4 {
+  uint2 h, m, l;
+};
+__device__ __forceinline__ Parts4 split_parts(f32x4 x) {
+  uint32_t hb[4], mb[4], lb[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    hb[i] = __float_as_uint(x[i]) & 0xffff0000u;
+    const float rest = x[i] - __uint_as_float(hb[i]);          // exact
+    mb[i] = __float_as_uint(rest) & 0xffff0000u;
+    lb[i] = __float_as_uint(rest - __uint_as_float(mb[i]));     // exact, low 16 bits zero
+  }
+  auto pk = [](uint32_t e0, uint32_t e1) { return (e0 >> 16) | (e1 & 0xffff0000u); };
+  return {{pk(hb[0], hb[1]), pk(hb[2], hb[3])}, {pk(mb[0], mb[1]), pk(mb[2], mb[3])},
+          {pk(lb[0], lb[1]), pk(lb[2], lb[3])}};
+}
+__device__ __forceinline__ bf16x8 join8(uint2 a, uint2 b) {
+  return __builtin_bit_cast(bf16x8, uint4{a.x, a.y, b.x, b.y});
+}
 
 // This workgroup's (row, 64-position chunk) item, and in a batch its chunk's arguments put into `a` and its
 // index into zc; false for a workgroup past the items.  Workgroups go round-robin over the 8 XCDs: XCD x
@@ -471,7 +493,7 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
         } else {
           mask(sum_ok);
         }
-        bf16x8 hi[HW], lo[HW];
+        bf16x8 hi[HW], mid[HW], lo[HW];
 #pragma unroll
         for (int u = 0; u < HW; ++u) {
           float mx = fmaxf(fmaxf(fmaxf(s[u][0][0], s[u][0][1]), fmaxf(s[u][0][2], s[u][0][3])),
@@ -497,10 +519,11 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
               const float e = __builtin_amdgcn_exp2f(s[u][tt][i] - mr);   // exp2(-inf) = 0
               s[u][tt][i] = e;
               lsum[u] += e;
-              const __bf16 h = (__bf16)e;
-              hi[u][4 * tt + i] = h;
-              lo[u][4 * tt + i] = (__bf16)(e - (float)h);
             }
+          const Parts4 x0 = split_parts(s[u][0]), x1 = split_parts(s[u][1]);
+          hi[u] = join8(x0.h, x1.h);
+          mid[u] = join8(x0.m, x1.m);
+          lo[u] = join8(x0.l, x1.l);
         }
         if (!page_bad) {
 #pragma unroll
@@ -513,6 +536,7 @@ page_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatc
 #pragma unroll
               for (int u = 0; u < HW; ++u) {
                 o[u][mt][half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi[u], o[u][mt][half], 0, 0, 0);
+                o[u][mt][half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, mid[u], o[u][mt][half], 0, 0, 0);
                 o[u][mt][half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo[u], o[u][mt][half], 0, 0, 0);
               }
             }

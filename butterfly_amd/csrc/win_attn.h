@@ -6,9 +6,9 @@
 // 16-slot tile of routed summaries.  Two phases share one LDS buffer of 208 rows:
 //   * K staged; each wave (16 query rows, HW heads) scores its nine window tiles and the summary tile
 //     (S^T = K Q^T, one K fragment read for the wave's heads), one maximum and one sum per row in fp32
-//     registers, P = hi + lo in two bf16 parts;
+//     registers, P = hi + mid + lo exactly in three bf16 parts;
 //   * V, requested with K and held in registers until every wave is done with K, staged in the same
-//     rows; O^T = V^T P^T tile by tile (one V fragment read for HW heads times two parts), stored as
+//     rows; O^T = V^T P^T tile by tile (one V fragment read for HW heads times three parts), stored as
 //     each 64 columns are done.
 // No running softmax: one maximum per row and chunk, no rescaling, and no output accumulators held
 // across the keys (page_attn_kernel holds D / 4 registers a head and runs 7 barriers a unit; 3 here).
@@ -201,7 +201,7 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
 
   // ---- scores and softmax: key 4 lg + i of tile t (window tiles: positions pw - 128 + 16 t .., rows
   // 16 (qwave + t) ..; tile 9: the summary slots)
-  bf16x8 hi[HW][5], lo[HW][5];
+  bf16x8 hi[HW][5], mid[HW][5], lo[HW][5];
   float inv[HW];
   const int wlo = max(max(qp - a.W + 1, a.key_lo), 0);
   const int qcut = max(0, (a.token_cutoff ? qp : qblk * a.bs) - a.W + 1);
@@ -258,18 +258,26 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
       const float nm = mx == -INFINITY ? 0.f : -mx * sl2;
       float l = 0.f;
 #pragma unroll
-      for (int t = 0; t < 10; ++t)
+      for (int pr = 0; pr < 5; ++pr) {
+        Parts4 x[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float e = 0.f;
+        for (int tt = 0; tt < 2; ++tt) {
+          const int t = 2 * pr + tt;
+          f32x4 e = {0.f, 0.f, 0.f, 0.f};
           if (t < NT) {
-            e = __builtin_amdgcn_exp2f(fmaf(s[u][t][i], sl2, nm));
-            l += e;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              e[i] = __builtin_amdgcn_exp2f(fmaf(s[u][t][i], sl2, nm));
+              l += e[i];
+            }
           }
-          const __bf16 h = (__bf16)e;
-          hi[u][t / 2][(t % 2) * 4 + i] = h;
-          lo[u][t / 2][(t % 2) * 4 + i] = (__bf16)(e - (float)h);
+          x[tt] = split_parts(e);
         }
+        hi[u][pr] = join8(x[0].h, x[1].h);
+        mid[u][pr] = join8(x[0].m, x[1].m);
+        lo[u][pr] = join8(x[0].l, x[1].l);
+        __builtin_amdgcn_sched_barrier(0);      // two tiles at a time: the parts take the scores' registers
+      }
       l = col_sum4(l);
       if constexpr (MODE == kPageFused) {
         inv[u] = 1.f / fmaxf(l, 1e-30f);
@@ -350,6 +358,7 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
 #pragma unroll
           for (int u = 0; u < HW; ++u) {
             o[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi[u][pr], o[u], 0, 0, 0);
+            o[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, mid[u][pr], o[u], 0, 0, 0);
             o[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo[u][pr], o[u], 0, 0, 0);
           }
         }
@@ -366,12 +375,12 @@ win_attn_kernel(PageArgs a_in, std::conditional_t<kBatch, PageBatch, PageNoBatch
             const bf16x4 x = *reinterpret_cast<const bf16x4*>(Vs + r * D + (unit ^ (2 * vrow_swizzle<D>(r))) * 4);
 #pragma unroll
             for (int u = 0; u < HW; ++u) {
-              float p = 0.f;
+              // (times an infinity or NaN: the high part of the weight says all that its value does)
+              unsigned word = 0;
 #pragma unroll
-              for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                  p = pick == 4 * t + i ? (float)hi[u][t / 2][(t % 2) * 4 + i] + (float)lo[u][t / 2][(t % 2) * 4 + i] : p;
+              for (int w32 = 0; w32 < 20; ++w32)
+                word = pick >> 1 == w32 ? __builtin_bit_cast(page_u32x4, hi[u][w32 / 4])[w32 % 4] : word;
+              float p = __uint_as_float(pick & 1 ? word & 0xffff0000u : word << 16);
               p = __shfl(p, src);
 #pragma unroll
               for (int e = 0; e < 4; ++e) {

@@ -3,7 +3,7 @@ values near the type's largest, against a 64-bit softmax per row.
 
 One call of every shape here has at least 256 workgroups, from which on such windows run on that kernel; streamed
 batches take it whatever their size.  Finite results are off by the output's rounding to bf16 (half an ulp, at most
-2^-8 of the value) and by the weights' 16 bits and fp32 arithmetic (below 1e-5 of values of up to 5).
+2^-8 of the value) and by fp32 arithmetic (below 1e-5 of values of up to 5).
 """
 from __future__ import annotations
 
@@ -84,8 +84,8 @@ def test_infinities_and_nans_stay_with_their_rows(case):
             assert torch.equal(torch.isposinf(out), torch.isposinf(want)), (bi, h)
             assert torch.equal(torch.isneginf(out), torch.isneginf(want)), (bi, h)
             fin = torch.isfinite(want)
-            # where 3e38 takes part, its weight's 16 bits are the measure
-            big = 3e38 * 2.0 ** -16 if kv == 4 and bi == 0 else 0.0
+            # where 3e38 takes part, its weight's fp32 rounding is the measure (scores of up to 8: below 2^-20)
+            big = 3e38 * 2.0 ** -20 if kv == 4 and bi == 0 else 0.0
             room = BF16_ROUNDING * want.abs() + ABS + big * (torch.arange(d) == 7)
             assert ((out - want).abs() <= room)[fin].all(), (bi, h)
             seen += int((~fin).sum())
@@ -132,3 +132,50 @@ def test_streamed_batches_keep_them_too(d, hq, hkv, bs, lens):
             assert ((out - want).abs() <= BF16_ROUNDING * want.abs() + ABS)[fin].all(), (c, h)
             seen += int((~fin).sum())
     assert seen > 100
+
+
+# kind, hq, hkv, t, d, W: win_attn_kernel with one and two heads a wave and four a workgroup, page_attn_kernel (small
+# grids, W above 128) in its splits, the window stream, and the dense summary stream (every earlier block of 16)
+WEIGHTS = [("call", 4, 4, 4160, 64, 128), ("call", 8, 4, 4160, 128, 100), ("call", 12, 4, 4160, 256, 128),
+           ("call", 2, 2, 1000, 128, 128), ("call", 8, 2, 1000, 256, 200), ("call", 16, 4, 4160, 128, 256),
+           ("call", 2, 1, 9000, 64, 256), ("window", 8, 4, 4160, 128, 128), ("window", 4, 4, 2000, 64, 64),
+           ("dense", 8, 2, 2000, 128, 1), ("dense", 4, 4, 2000, 64, 1)]
+
+
+@pytest.mark.parametrize("kind,hq,hkv,t,d,w", WEIGHTS)
+def test_weights_keep_fp32_precision(kind, hq, hkv, t, d, w):
+    """Values that cancel under a row's weights leave the weights' own error: some queries with windows apart, each
+    with four keys chosen so that the weighted sum of every column is next to zero.  Scores near zero keep an fp32
+    weight within about 2^-23 of itself, and sums of random sign come to 2^-22.5 of size = sqrt(sum (p v)^2); weights
+    of 16 bits miss by 2^-19.5 of size (rms)."""
+    g, bs = hq // hkv, 16 if kind == "dense" else 128
+    q, k, v = _rand(1, 1, hq, t, d) * 0.05, _rand(2, 1, hkv, t, d), _rand(3, 1, hkv, t, d)
+    n = t // bs if kind == "dense" else 0
+    ks, vs = _rand(4, 1, hkv, max(n, 1), d), _rand(5, 1, hkv, max(n, 1), d)
+    keys, vals, rows = (ks, vs, [t - 1]) if kind == "dense" else (k, v, range(w + 70, t, w + 113))
+    picked = []
+    for kv in range(hkv):
+        for i, r in enumerate(rows):
+            h = kv * g + i % g
+            lo, hi = (0, r // bs) if kind == "dense" else (r - w + 1, r + 1)
+            p = torch.softmax((keys[0, kv, lo:hi].double() @ q[0, h, r].double()) * d ** -0.5, -1)[:, None]
+            x = vals[0, kv, lo:hi].double()
+            for key in (hi - lo) * torch.tensor([1, 3, 6, 8]) // 9:
+                x[key] = 0
+                x[key] = (-(p * x).sum(0) / p[key]).bfloat16().double()
+            vals[0, kv, lo:hi] = x.bfloat16()
+            picked.append((h, r, (p * x).sum(0), (p * x).pow(2).sum(0).sqrt()))
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    if kind == "call":
+        lay = bf.build_block_butterfly_layout(seq_len=t, block_size=bs, num_key_value_heads=hkv, num_key_value_groups=g,
+                                              layer_idx=0, local_window_blocks=0, sink_count=0, partner_count=0,
+                                              partner_rule="xor")      # no summaries
+        got = bf.compressed_butterfly_attention(qd, kd, vd, layout=lay, local_window_tokens=w)[0]
+    elif kind == "window":
+        got = bf.swa_stream_attention(qd, kd, vd, n_win=w, scale=d ** -0.5)[0]
+    else:
+        got = bf.compressed_stream_attention(qd, ks.cuda(), vs.cuda(), block_size=bs, scale=d ** -0.5)[0]
+    got = got[0].cpu().double()
+    worst = max(((got[h, r] - want).abs() - BF16_ROUNDING * want.abs()).div(size).max().item()
+                for h, r, want, size in picked)
+    assert worst <= 2.0 ** -20

@@ -1660,6 +1660,10 @@ static void launch_win_batch(PageArgs a, PageBatch cb, int d, int nchunks_max, h
   };
   const int64_t units = (int64_t)nchunks_max * cb.nch * a.batch * a.hkv;
   if (d == 256) {
+    // Four heads from 128 workgroups on (below, the split in two halves a unit's chain).  Streams of 20480 tokens,
+    // window 128, two heads and four a workgroup, us: 12/3 heads in chunks of 512 (240 workgroups of four) 277 and
+    // 249, 16/4 in chunks of 256 (160) 383 and 361, 16/2 in chunks of 192 (120) 568 and 615, 4/1 in chunks of 512
+    // (80) level.
     if (gsz >= 3 && units * ((gsz + 3) / 4) >= 128) go(win_attn_kernel<256, 2, 2, kPageFused, true>, 4, 2);
     else go(win_attn_kernel<256, 1, 2, kPageFused, true>, 2, 2);
   } else if (d == 128) {

@@ -447,7 +447,9 @@ static inline void launch_win_attn(PageArgs a, int d, hipStream_t stream) {
   };
   const bool two = gsz >= 2;
   if (d == 256) {
-    if (gsz >= 3 && units * ((gsz + 3) / 4) >= 256) go(win_attn_kernel<256, 2, 2, MODE>, 4, 2);
+    // four heads a workgroup on whatever grid win_fills lets through: 16/4 heads, window 128, 2100 / 3840 tokens
+    // (132 / 240 such workgroups) 28.1 / 30.5 us a call, 35.0 / 38.8 with two heads in twice as many
+    if (gsz >= 3) go(win_attn_kernel<256, 2, 2, MODE>, 4, 2);
     else go(win_attn_kernel<256, 1, 2, MODE>, 2, 2);
   } else if (d == 128) {
     if (two) go(win_attn_kernel<128, 2, 1, MODE>, 2, 1);

@@ -52,7 +52,7 @@ def _prefill64(q, k, v, ks, vs, ref, w, bs):
 # workgroup at d = 256, blocks of half a page, lengths off the page and the 16-row tile
 CASES = [(4, 8, 8, 533, 64, 64, 65), (4, 16, 8, 530, 64, 32, 128), (4, 8, 8, 560, 128, 64, 100),
          (3, 24, 8, 700, 128, 128, 128), (4, 16, 8, 521, 128, 64, 127), (4, 8, 8, 530, 256, 64, 128),
-         (2, 24, 8, 1040, 256, 128, 96)]
+         (2, 24, 8, 1040, 256, 128, 96), (2, 32, 8, 530, 256, 64, 128)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c))

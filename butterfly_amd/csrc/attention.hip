@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(64) attn_generic_kernel(AttnArgs a) {
 // (all but |al bl| < 2^-28 |a b|), the softmax exponent in one fma, infinities and NaN key by key
 // (f32_rows_plainly).  Over 3 draws of 5 shapes against 64 bits: rms 3.7e-8..5.5e-8 where the generic
 // kernel has 4.9e-8..7.1e-8, the largest single error 1.75e-6 against 1.73e-6.  Calls of 4096 tokens, 8/2
-// heads of d 128: W = 128 303 -> 55 us, W = 65 184 -> 55 us; one row over such a cache, W = 128,
+// heads of d 128: W = 128 280 -> 41 us, W = 65 165 -> 39 us; one row over such a cache, W = 128,
 // 84 -> 44 us (the calls' host part included): the rule needs no lower limit on the rows.
 // Positions and ring slots are 32-bit (the host sends only caches and rings below 2^30 rows here).
 constexpr int kF32MaxKcap = 16;
@@ -1497,7 +1497,7 @@ static int chunk_blocks_max(int bs) { return bs % kPageRows == 0 ? 1 : kPageRows
 // Whether the paged kernel takes a bf16 launch over contiguous positions: its summary page holds 64
 // slots (the routed rows of every block that 64 positions touch), a ring page may wrap once,
 // positions are 32-bit.  It replaces the generic kernel wherever it can run: the one-shot call over
-// 2 x 10007 tokens, 16 query heads over 4 of d 128, W 128 took 1711 us there and 109 us here (78 on
+// 2 x 10007 tokens, 16 query heads over 4 of d 128, W 256 takes 3185 us there and 152 us here (W 128 82 on
 // win_attn_kernel, which has the windows of 65..128 where the grid fills the chip).
 static bool page_path(const AttnArgs& a, int blocks) {
   return (a.d == 64 || a.d == 128 || a.d == 256) && a.W + (int64_t)a.kcap <= kGenericMaxKeys &&
@@ -1999,7 +1999,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // the attention's halo lies in (ring_disjoint).  With the default ring (1408 rows for 512-token chunks
   // and 128-token windows) that is ten chunks a launch instead of one: 20011 tokens of d 256, 16
   // query heads over 4, window 128: 1812 us a stream with a launch per chunk, 407 so, both on
-  // page_attn_kernel (288 on win_attn_kernel).
+  // page_attn_kernel (309 to 312 on win_attn_kernel, with weights in three parts instead of two).
   struct Batch {
     int64_t first = 0, count = 0, total = 0;
     AttnArgs args[kMaxUpdateParts];
@@ -2020,8 +2020,8 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // chunk per batch leaves.  A W <= 64 call whose chunks share batches under the length rule keeps
   // that rule alone (its batches copy only their tails), and so does one with a chunk off the page grid,
   // which no wide batch holds: 9000 tokens of d 256 in chunks of 700, 251 us, 262 with the copies
-  // alone.  In chunks of 512, 20000 tokens of d 256, 16/4 heads, window 64: 630 us by length, 327 wide;
-  // of 1024, 30000 tokens of d 64, 8/4 heads: 400 and 203.
+  // alone.  In chunks of 512, 20000 tokens of d 256, 16/4 heads, window 64: 607 us by length, 318 wide;
+  // of 1024, 30000 tokens of d 64, 8/4 heads: 398 and 197.
   bool wide = paged || s.offset % kPage == 0;
   for (int64_t c = 0; !paged && c + 1 < n_chunks; ++c)
     if (chunk_len[c] + chunk_len[c + 1] <= budget || chunk_len[c] % kPage != 0) wide = false;

@@ -715,12 +715,14 @@ def chunked_prefill(core: ButterflyAttentionCore, chunks, cache: CompressedKVCac
 
 
 # Chunks per bfly_stream_chunks call: a first run of 8, then each run about 1.3 times the one
-# before, in whole batches of the native loop (its batches hold at most 10 chunks and half the ring
-# minus two pages), up to 256.  The host prepares a call's chunks (about 2 us each) before its first
+# before, in whole batches of the native loop as its length rule makes them (at most 10 chunks and
+# half the ring minus two pages), up to 256.  Chunks on the page grid whose window lies above 64, or
+# of which no two fit by length, go in batches of more than that, up to 10, and a run of them may
+# end in a smaller batch.  The host prepares a call's chunks (about 2 us each) before its first
 # launch, while the GPU works through the call before (about 3 us per chunk, of which about 2 are
 # still queued when that call returns); a run 1.3 times the last is ready before that queue drains,
-# where 1.5 times left the GPU waiting at every call boundary.  A call rarely ends in a small batch,
-# whose attention launch runs alone.
+# where 1.5 times left the GPU waiting at every call boundary.  Under the length rule a call rarely
+# ends in a small batch, whose attention launch runs alone.
 _STREAM_GROWTH = 1.3
 _STREAM_RUN_MAX = 256
 _STREAM_BATCH_CAP = 10

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import re
+import threading
 from pathlib import Path
 
 import pytest
@@ -219,3 +220,23 @@ def test_add_rms_norm_q4_gemv_validates_before_launch(args, msg):
     *head, out, st = args
     assert lib.bfly_add_rms_norm_q4_gemv_silu(*head, head[7], out, st) == _native.ERR_INVALID
     assert msg in lib.bfly_last_error()
+
+
+def test_messages_are_per_thread():
+    lib, seen = _native.lib(), {}
+    s = C.c_int32()
+
+    def other(rule):
+        seen[rule, "before"] = lib.bfly_last_error()
+        lib.bfly_stage_meta(8, 0, rule, C.byref(s), C.byref(s), C.byref(s))
+        seen[rule, "after"] = lib.bfly_last_error()
+
+    assert lib.bfly_stage_meta(8, 0, 99, C.byref(s), C.byref(s), C.byref(s)) == _native.ERR_INVALID
+    mine = lib.bfly_last_error()
+    assert b"99" in mine
+    for rule in (77, 88):
+        t = threading.Thread(target=other, args=(rule,))
+        t.start()
+        t.join()
+        assert seen[rule, "before"] == b"" and str(rule).encode() in seen[rule, "after"]
+    assert lib.bfly_last_error() == mine

@@ -1999,7 +1999,7 @@ extern "C" int bfly_stream_chunks(int64_t n_chunks, const void* const* q, const 
   // the attention's halo lies in (ring_disjoint).  With the default ring (1408 rows for 512-token chunks
   // and 128-token windows) that is ten chunks a launch instead of one: 20011 tokens of d 256, 16
   // query heads over 4, window 128: 1812 us a stream with a launch per chunk, 407 so, both on
-  // page_attn_kernel (309 to 312 on win_attn_kernel, with weights in three parts instead of two).
+  // page_attn_kernel (306 on win_attn_kernel, with weights in three parts instead of two).
   struct Batch {
     int64_t first = 0, count = 0, total = 0;
     AttnArgs args[kMaxUpdateParts];

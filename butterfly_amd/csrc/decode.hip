@@ -952,7 +952,7 @@ __device__ __forceinline__ void dec_pool32(const DecodeArgs& a, const DecState32
 // block (the same values), so none reads what another writes in the launch.
 // kWin: window rows staged, 64 or (host-counter steps) 128.  The wide form stages 144 keys, nine
 // score tiles and five PV k-steps, and keeps P whole, all 24 bits of the fp32 value, in three bf16 parts.  One
-// sequence, 16/4 heads of 128, window 128, a step with its append: 19.0 us a call (19.0 with P in two parts, whose
+// sequence, 16/4 heads of 128, window 128, a step with its append: 19.0 us a call, host-bound (19.0 with P in two parts, whose
 // 16 or 17 bits moved outputs by a bf16 step; as an update launch and a paged attention launch 22.7, with a generic
 // attention launch 81.6).  It is a chain of latencies: loads, nine score tiles, one softmax, PV.
 template <int D, bool kStep, bool kQkn = false, int kOS = 0, int kWin = kDecMaxWin>

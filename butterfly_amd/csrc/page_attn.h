@@ -30,8 +30,8 @@
 // HBM traffic is Q and O once and the K/V pages about once per XCD (consecutive units of one kv
 // head share their pages in an L2).  Measured, whole calls: 2 x 10007 tokens, 16/4 heads of d 128,
 // W 256 3185 us on the generic kernel, 152 here (141 with P in two parts, 17 of its 24 bits); 512 rows over
-// 32k tokens 135 and 31 to 33 (compressor included); window stream, dense summaries and merge over 8192 tokens,
-// 8/2 heads 680 and 47 to 50.
+// 32k tokens 135 and 28 to 29 (compressor included); window stream, dense summaries and merge over 8192 tokens,
+// 8/2 heads 680 and 45.
 #pragma once
 
 #include "bfly_topology.h"

@@ -10,7 +10,7 @@
 //
 // bf16 with head_dim 64, 128 or 256 runs on the paged MFMA kernel (page_attn.h): window stream,
 // dense summaries and merge over 8192 tokens, 8 query heads over 2 of d 128, took 680 us on
-// stream_kernel and take 47 to 50 us there.
+// stream_kernel and take 45 us there.
 //
 // stream_kernel (fp32, other head dims): one wave per (batch, query head, query).  Keys are visited in
 // groups of 64 (one per lane) with a running max and rescaled accumulators, so

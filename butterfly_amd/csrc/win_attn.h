@@ -21,7 +21,7 @@
 // What bounds it: the chain request, scores, softmax, V, store within a workgroup (two of them per CU at
 // d = 128), with the VALU about 36% and the matrix cores about 25% busy.  2 x 10007 tokens, 16/4 heads of d 128,
 // W 128, with the compressor's 8 us: 82 us a call (40 by bytes); 20011 tokens of d 256 streamed in chunks of 512:
-// 309 to 312.  With P in two parts, 17 of its 24 bits: 78 and 288 here, 109 and 407 on page_attn_kernel.
+// 306.  With P in two parts, 17 of its 24 bits: 78 and 288 here, 109 and 407 on page_attn_kernel.
 #pragma once
 
 #include "page_attn.h"
